@@ -941,84 +941,145 @@ __global__ __launch_bounds__(256) void gemm_dma128_kernel(GemmArgs g) {
 }
 
 // Few rows (M <= 64) against k-contiguous b (b^T rows, x @ w.t(): a linear layer on a few
-// tokens).  The product reads b once and is bound by streaming it, which the 128-wide tiles
-// spread over too few workgroups (N / 128).  Here a workgroup owns 32 columns (32 rows of
-// b^T) and one 32-row block of a (blockIdx.y); its eight waves take contiguous eighths of K
-// and load their MFMA fragments straight from memory (a lane's row of a, or column of b, at
-// k 8 (lane / 32) .. + 7 of each 16-deep step: 16 bytes per operand), four steps in flight.
-// The eight partial 32 x 32 tiles are then summed through LDS and finished element by
-// element (alpha, round, beta c, any out type).  One row block per workgroup rather than
-// both in one: 64 x 4096 x 4096 fp16 18.8 against 26.9 us (more workgroups, half the work
-// each).
+// tokens).  The product reads b once and is bound by streaming it.  A workgroup owns 16 NB
+// columns (rows of b^T) and 16 MB rows of a; its NW waves take the 64-deep chunks of K in
+// turn (wave w chunks w, w + NW, ...) and load their MFMA fragments straight from memory:
+// v_mfma_f32_16x16x32 takes from lane l row (column) l % 16 at k 8 (l / 16) .. + 7, so one
+// 16-byte load per lane covers 64 contiguous bytes of 16 rows and a chunk's two loads the
+// row's whole 128-byte line.  D chunks are in flight per wave.  The NW partial tiles are
+// summed through LDS and finished element by element (alpha, round, beta c, any out type).
+// Rows need no alignment (16-byte loads of 2-byte aligned data), so K and the row strides
+// may be anything: only the last, partial chunk of K is loaded element by element.  Rows
+// past M and columns past N read row 0 and are never stored.
 namespace skinny {
-constexpr int NW = 8, STEPS = 4;
+constexpr int KC = 64;  // k per chunk: one 128-byte line of a row
+struct __attribute__((packed, aligned(2))) unaligned16 {
+  u32x4 v;
+};
+template <typename T>
+struct mma16;
+template <>
+struct mma16<f16_t> {
+  __device__ __forceinline__ static floatx4 mma(u32x4 a, u32x4 b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
+  }
+};
+template <>
+struct mma16<bf16_t> {
+  __device__ __forceinline__ static floatx4 mma(u32x4 a, u32x4 b, floatx4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
+                                                   0);
+  }
+};
 }  // namespace skinny
 
-template <typename T>
-__global__ __launch_bounds__(64 * skinny::NW) void gemm_skinny_kernel(GemmArgs g) {
-  constexpr int MB = 1;  // 32-row blocks of a per workgroup
-  __shared__ float part[skinny::NW * MB * 16 * 64];
-  const int64_t m0 = 32 * (int64_t)blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63;
+template <typename T, int MB, int NB, int NW, int D>
+__global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(GemmArgs g) {
+  __shared__ float part[NW * MB * NB * 4 * 64];
+  const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, kg = (lane >> 4) * 8;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t n0 = (int64_t)blockIdx.x * 32;
-  const int nsteps = (int)((g.K + 15) / 16);
-  const int per = (nsteps + skinny::NW - 1) / skinny::NW;
-  const int s0 = wave * per, s1 = min(nsteps, s0 + per);
-  const int kl = 8 * (lane >> 5);
-  const int64_t n = n0 + (lane & 31);
-  const bool n_ok = n < g.N;
-  const uint16_t* brow = (const uint16_t*)g.b + (n_ok ? n : 0) * g.sb_n + kl;
-  const uint16_t* arow[MB];
-  bool m_ok[MB];
+  const int64_t m0 = (int64_t)blockIdx.y * (16 * MB), n0 = (int64_t)blockIdx.x * (16 * NB);
+  const uint16_t *arow[MB], *brow[NB];
 #pragma unroll
   for (int i = 0; i < MB; ++i) {
-    const int64_t m = m0 + 32 * i + (lane & 31);
-    m_ok[i] = m < g.M;
-    arow[i] = (const uint16_t*)g.a + (m_ok[i] ? m : 0) * g.sa_m + kl;
+    const int64_t m = m0 + 16 * i + r16;
+    arow[i] = (const uint16_t*)g.a + (m < g.M ? m : 0) * g.sa_m + kg;
   }
-  typedef typename mfma_traits<T>::frag frag;
-  // Step s: this lane's 8 k of a row of each a block and of a column of b (zeros past M, N, K;
-  // K is a multiple of 8, so a lane's 8 k are all inside or all outside).
-  auto load = [&](int st, frag (&fa)[MB], frag& fb) {
-    const int64_t k = (int64_t)st * 16;
-    const bool k_ok = k + kl < g.K;
-    const u32x4 z = {0u, 0u, 0u, 0u};
-    fb = __builtin_bit_cast(frag, n_ok && k_ok ? *(const u32x4*)(brow + k) : z);
 #pragma unroll
-    for (int i = 0; i < MB; ++i) fa[i] = __builtin_bit_cast(frag, m_ok[i] && k_ok ? *(const u32x4*)(arow[i] + k) : z);
-  };
-  floatx16 acc[MB];
+  for (int j = 0; j < NB; ++j) {
+    const int64_t n = n0 + 16 * j + r16;
+    brow[j] = (const uint16_t*)g.b + (n < g.N ? n : 0) * g.sb_n + kg;
+  }
+  floatx4 acc[MB][NB];
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
-  frag fa[skinny::STEPS][MB], fb[skinny::STEPS];
+    for (int j = 0; j < NB; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  const int chunks = (int)(g.K / skinny::KC);  // whole chunks of K
+  const int mine = chunks > wave ? (chunks - wave + NW - 1) / NW : 0;
+  u32x4 fa[D][2][MB], fb[D][2][NB];
+  auto load = [&](int c, int slot) {
+    const int64_t k = (int64_t)(wave + c * NW) * skinny::KC;
 #pragma unroll
-  for (int j = 0; j < skinny::STEPS; ++j)
-    if (s0 + j < s1) load(s0 + j, fa[j], fb[j]);
-  for (int st = s0; st < s1; st += skinny::STEPS) {
+    for (int h = 0; h < 2; ++h) {
 #pragma unroll
-    for (int j = 0; j < skinny::STEPS; ++j) {
-      if (st + j < s1) {
+      for (int j = 0; j < NB; ++j) fb[slot][h][j] = ((const skinny::unaligned16*)(brow[j] + k + 32 * h))->v;
 #pragma unroll
-        for (int i = 0; i < MB; ++i) acc[i] = mfma_traits<T>::mma(fa[j][i], fb[j], acc[i]);
-        if (st + j + skinny::STEPS < s1) load(st + j + skinny::STEPS, fa[j], fb[j]);
+      for (int i = 0; i < MB; ++i) fa[slot][h][i] = ((const skinny::unaligned16*)(arow[i] + k + 32 * h))->v;
+    }
+  };
+  auto mul = [&](int slot) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[i][j] = skinny::mma16<T>::mma(fa[slot][h][i], fb[slot][h][j], acc[i][j]);
+  };
+  // No load of the pipelined loop is conditional: past a branch that may load, the compiler's
+  // wait for an older chunk would be a wait for every load.
+  if (mine >= D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(d, d);
+    int c = 0;
+    for (; c + 2 * D <= mine; c += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        mul(d);
+        load(c + D + d, d);
       }
     }
+    const int rest = mine - c - D;
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      mul(d);
+      if (d < rest) load(c + D + d, d);
+    }
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d)
+      if (d < rest) mul(d);
+  } else {
+    for (int c = 0; c < mine; ++c) {
+      load(c, 0);
+      mul(0);
+    }
   }
-  // Sum the eight waves' partial tiles: acc[i][r] of lane l is C[32 i + acc_row(r, l)][n0 + l % 32].
+  // The partial last chunk, by the wave whose turn it is: values past K are zeros.
+  const int64_t k_tail = (int64_t)chunks * skinny::KC;
+  if (k_tail < g.K && wave == chunks % NW) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int64_t left = g.K - (k_tail + 32 * h + kg);  // k of this lane inside K
+      auto partial = [&](const uint16_t* row) {
+        const uint16_t* p = row + k_tail + 32 * h;
+        if (left >= 8) return ((const skinny::unaligned16*)p)->v;
+        u32x4 v = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (u < left) v[u >> 1] |= (uint32_t)p[u] << (16 * (u & 1));
+        return v;
+      };
+#pragma unroll
+      for (int j = 0; j < NB; ++j) fb[0][h][j] = partial(brow[j]);
+#pragma unroll
+      for (int i = 0; i < MB; ++i) fa[0][h][i] = partial(arow[i]);
+    }
+    mul(0);
+  }
+  // Sum the partial tiles: acc[i][j][r] of lane l is C[16 i + 4 (l / 16) + r][16 j + l % 16].
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) part[((wave * MB + i) * 16 + r) * 64 + lane] = acc[i][r];
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) part[(((wave * MB + i) * NB + j) * 4 + r) * 64 + lane] = acc[i][j][r];
   __syncthreads();
-  for (int e = tid; e < MB * 16 * 64; e += 64 * skinny::NW) {
-    const int l = e & 63, ir = e >> 6, i = ir >> 4, r = ir & 15;
+  for (int e = tid; e < MB * NB * 256; e += 64 * NW) {
+    const int l = e & 63, r = (e >> 6) & 3, ij = e >> 8, i = ij / NB, j = ij % NB;
     float v = 0.0f;
 #pragma unroll
-    for (int w = 0; w < skinny::NW; ++w) v += part[((w * MB + i) * 16 + r) * 64 + l];
-    const int64_t row = m0 + 32 * i + acc_row(r, l), col = n0 + (l & 31);
+    for (int w = 0; w < NW; ++w) v += part[w * (MB * NB * 256) + e];
+    const int64_t row = m0 + 16 * i + 4 * (l >> 4) + r, col = n0 + 16 * j + (l & 15);
     if (row < g.M && col < g.N) {
       float out = g.alpha * round_through(v, g.round_dtype);
       if (g.c) out += g.beta * load_c<false>(g, row * g.sc_m + col * g.sc_n);
@@ -1451,20 +1512,44 @@ static int gemm16_launch(GemmArgs g, hipStream_t stream, int config = 0) {
                          g.K >= 3 * 32 && !dma128_nn;
   const int64_t tiles128 = cdiv(g.M, 128) * cdiv(g.N, 128);
   const bool ok128 = (dma128_nn || dma128_bt) && out_vec && c_vec && g.N % 8 == 0 && tiles128 <= 0x7fffffffLL;
-  // gemm_skinny_kernel: at most 64 rows, a and b^T rows k-contiguous with 16-byte aligned rows.
-  const bool skinny = g.M <= 64 && g.sa_k == 1 && g.sb_k == 1 && g.sa_m >= 0 && g.sb_n > 0 && (uintptr_t)g.a % 16 == 0 &&
-                      (uintptr_t)g.b % 16 == 0 && g.sa_m % 8 == 0 && g.sb_n % 8 == 0 && g.K % 8 == 0 &&
-                      cdiv(g.N, 32) <= 0x7fffffffLL;
-  if ((config == 1 && !dma_ok) || (config == 2 && !fast) || (config == 4 && !ok128) || (config == 5 && !skinny))
+  // gemm_skinny_kernel: at most 64 rows, a and b^T rows k-contiguous, of any alignment and
+  // length (forced as configuration 5: 16-byte aligned rows, K a multiple of 8).
+  const bool skinny = g.M <= 64 && g.sa_k == 1 && g.sb_k == 1 && cdiv(g.N, 16) <= 0x7fffffffLL &&
+                      g.K / skinny::KC <= 0x7fffffffLL;
+  const bool skinny_forced = skinny && g.sa_m >= 0 && g.sb_n > 0 && (uintptr_t)g.a % 16 == 0 &&
+                             (uintptr_t)g.b % 16 == 0 && g.sa_m % 8 == 0 && g.sb_n % 8 == 0 && g.K % 8 == 0;
+  if ((config == 1 && !dma_ok) || (config == 2 && !fast) || (config == 4 && !ok128) || (config == 5 && !skinny_forced))
     return NT_ERR_INVALID;
-  // Default: up to 32 rows, or up to 64 with N <= 4096; past 32 rows with wide N the 128-wide
-  // tiles win (fp16, interleaved medians, few-rows / 128-wide / torch: 1 x 4096 x 4096
-  // 11.6 / 29.4 / 21.4 us; 16 x 4096 x 4096 14.8 / 30.3 / 19.9; 8 x 11008 x 4096 26.9 / 32.1 /
-  // 21.6; 64 x 4096 x 4096 18.8 / 32.6 / 21.4; 64 x 4096 x 11008 48.2 / 84.2 / 30.5; 33 x 11008 x
-  // 4096 47.6 / 33.1 / 21.7).
-  if (config == 5 || (config == 0 && skinny && (g.M <= 32 || g.N <= 4096))) {
-    const dim3 gridS((unsigned)cdiv(g.N, 32), (unsigned)cdiv(g.M, 32));
-    hipLaunchKernelGGL((gemm_skinny_kernel<T>), gridS, dim3(64 * skinny::NW), 0, stream, g);
+  // Up to 64 rows.  bf16 us with weights rotated past the caches, this kernel / what ran before
+  // (32 columns per workgroup with 32 bytes of a row per load, or the 128-wide tiles; for
+  // unaligned rows the element-wise loader) / torch: 1 x 4096 x 4096 7.6 / 16.0 / 19.3;
+  // 16 x 11008 x 4096 25.9 / 43.0 / 26.1; 7 x 3001 x 2050 5.9 / 1047 / 18.7;
+  // 32 x 4096 x 4096 14.3 / 25.5 / 18.6; 64 x 4096 x 4096 18.5 / 23.7 / 18.8;
+  // 64 x 4096 x 11008 46.6 / 62.4 / 34.1; 64 x 11008 x 4096 34.4 / 56.0 / 27.7.
+  // Up to 16 rows one block of 16 by 16 and sixteen waves (4 chunks in flight).  Past that the
+  // rows of a, which every workgroup reads again, cost as much as b's: 32 x 16 while that
+  // leaves no fewer workgroups than CUs (32 x 4096 x 4096: 14.3 against 18.4 us with 32 x 32),
+  // 32 x 32 blocks from 256 of those (64 x 4096 x 4096: 18.5 against 25.4 with 32 x 16), 64 x 64
+  // from 128 column blocks (64 x 11008 x 4096: 34.4 against 50.1 with 32 x 32).
+  if (config == 5 || (config == 0 && skinny)) {
+    auto go = [&](auto mb_c, auto nb_c, auto nw_c, auto d_c) {
+      constexpr int MB = decltype(mb_c)::value, NB = decltype(nb_c)::value, NW = decltype(nw_c)::value;
+      const dim3 gridS((unsigned)cdiv(g.N, 16 * NB), (unsigned)cdiv(g.M, 16 * MB));
+      hipLaunchKernelGGL((gemm_skinny_kernel<T, MB, NB, NW, decltype(d_c)::value>), gridS, dim3(64 * NW), 0, stream, g);
+    };
+    using C1 = std::integral_constant<int, 1>;
+    using C2 = std::integral_constant<int, 2>;
+    using C4 = std::integral_constant<int, 4>;
+    using C8 = std::integral_constant<int, 8>;
+    using C16 = std::integral_constant<int, 16>;
+    if (g.M <= 16)
+      go(C1{}, C1{}, C16{}, C4{});
+    else if (g.M > 32 && cdiv(g.N, 64) >= 128)
+      go(C4{}, C4{}, C8{}, C1{});
+    else if (g.M > 32 && 2 * cdiv(g.N, 32) >= 256)
+      go(C2{}, C2{}, C8{}, C2{});
+    else
+      go(C2{}, C1{}, C8{}, C4{});
     return launch_status();
   }
   if (config == 4 || (config == 0 && ok128 && tiles_m * tiles_n < DMA128_BELOW)) {

@@ -441,6 +441,27 @@ def test_gemm_few_rows(mnk, dtype):
     assert torch.allclose(out32, a.float() @ b.float(), atol=1e-3, rtol=1e-3)
 
 
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("mnk", ((1, 17, 63), (1, 15, 4097), (16, 1000, 130), (17, 33, 71), (33, 8200, 193),
+                                 (64, 4099, 1021), (49, 40, 2049)))
+def test_gemm_few_rows_unaligned(mnk, dtype):
+    # Rows of any length and alignment (odd K and row strides, 2-byte aligned starts): the last
+    # partial chunk of K must add nothing past K, where the buffers hold infinities.
+    m, n, k = mnk
+    abuf = torch.full((m, k + 3), float("inf"), dtype=dtype, device=DEV)
+    wbuf = torch.full((n, k + 5), float("inf"), dtype=dtype, device=DEV)
+    a, w = abuf[:, 1:k + 1], wbuf[:, 3:k + 3]
+    a.copy_(_randn((m, k), dtype, 116, 1.0 / math.sqrt(k)))
+    w.copy_(_randn((n, k), dtype, 117))
+    c = _randn((m, n), dtype, 118)
+    out = torch.empty((m, n), dtype=dtype, device=DEV)
+    kernels.gemm(a, w.t(), out, c=c, alpha=0.5, beta=2.0)
+    ref = 0.5 * (a.double() @ w.double().t().contiguous()) + 2.0 * c.double()
+    # the result's rounding, and fp32 sums of k products of about 1 / sqrt(k)
+    tol = 1e-2 if dtype == torch.bfloat16 else 2e-3
+    assert torch.allclose(out.double(), ref, atol=tol, rtol=tol)
+
+
 def test_gemm_few_rows_rejects_unfit_calls():
     from ninetoothed_amd.errors import KernelLaunchError
 
