@@ -357,7 +357,8 @@ int nt_attention_f32(const void* q, const int64_t* q_strides, const void* k, con
  * as nt_attention_f16/bf16 choose; 1 = the one-wave-per-SIMD pipelined kernel, head dim
  * 128 with unit d-stride and 16-byte aligned rows; 2 = the eight-wave kernel, same
  * conditions, any head dim up to 128 that is a multiple of 8 (padded with zeros to 64 or
- * 128); 3 = the four-wave kernels, any strides).  A forced
+ * 128); 3 = the four-wave kernels, any strides; 4 = the key-streaming kernel, conditions of
+ * 2).  A forced
  * configuration whose conditions do not hold returns NT_ERR_INVALID before launching.
  * Replaces the per-configuration launchers the reference's auto-tuner times over
  * BLOCK_SIZE_M/N (reference tests/test_attention.py:10-11,
@@ -370,6 +371,21 @@ int nt_attention_config_bf16(const void* q, const int64_t* q_strides, const void
                              const void* v, const int64_t* v_strides, void* o, const int64_t* o_strides,
                              int o_dtype, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D,
                              float q_scale, int causal, hipStream_t stream, int config);
+
+/* The same attention with a workspace (no counterpart in the reference): with few queries and
+ * few heads the keys of each query block are split over several workgroups, whose states
+ * (fp32) pass through `workspace`.  nt_attention_workspace_size gives the bytes it wants for
+ * these sizes (0: none); with none, too few, or one that is not 16-byte aligned, the keys are
+ * not split.  The workspace holds nothing between calls. */
+int64_t nt_attention_workspace_size(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D, int causal, int dtype);
+int nt_attention_ws_f16(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+                        const void* v, const int64_t* v_strides, void* o, const int64_t* o_strides,
+                        int o_dtype, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D,
+                        float q_scale, int causal, hipStream_t stream, void* workspace, int64_t workspace_bytes);
+int nt_attention_ws_bf16(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+                         const void* v, const int64_t* v_strides, void* o, const int64_t* o_strides,
+                         int o_dtype, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D,
+                         float q_scale, int causal, hipStream_t stream, void* workspace, int64_t workspace_bytes);
 
 /* ---------------------------------------------------------------------------
  * Generic kernels for programs that match none of the families above.  They replace

@@ -89,12 +89,19 @@ _SIGNATURES = {
                                      _P, _I)
         for t in ("f16", "bf16")
     },
+    **{
+        f"nt_attention_ws_{t}": (_P, _I64P, _P, _I64P, _P, _I64P, _P, _I64P, _I, _I64, _I64, _I64, _I64, _I64, _F, _I, _P,
+                                 _P, _I64)
+        for t in ("f16", "bf16")
+    },
+    "nt_attention_workspace_size": (_I64,) * 5 + (_I, _I),
     "nt_rtc_compile": (ctypes.c_char_p, ctypes.c_char_p, ctypes.POINTER(_P), _I64P, ctypes.c_char_p, _I64),
     "nt_rtc_free": (_P,),
     "nt_rtc_load": (_P, ctypes.c_char_p, ctypes.POINTER(_P)),
     "nt_rtc_launch": (_P, ctypes.c_uint32, ctypes.c_uint32, ctypes.POINTER(_P), _P),
 }
-_RESTYPES = {"nt_conv2d_workspace_size": ctypes.c_int64, "nt_rtc_free": None}
+_RESTYPES = {"nt_conv2d_workspace_size": ctypes.c_int64, "nt_attention_workspace_size": ctypes.c_int64,
+             "nt_rtc_free": None}
 
 _lock = threading.Lock()
 _library = None

@@ -21,6 +21,8 @@
 // MFMA-bound: 4 * B * H * Sq * Sk * D flops per launch (half of that when causal).
 #include "mfma_core.h"
 
+#include <algorithm>
+
 namespace nt {
 
 constexpr int AT_BM = 128;  // queries per workgroup
@@ -34,6 +36,10 @@ struct AttnArgs {
   int64_t B, H, Sq, Sk, D;
   float q_scale;
   int causal, o_dtype, q_blocks;
+  // attention_keys_kernel: workgroups per query block, and (more than one) their states in the
+  // workspace: O [split][head][query][DM] and (max, sum) [split][head][query][2].
+  int splits;
+  float *part_o, *part_ml;
 };
 
 // Workgroup id -> (query block, batch*head).  The dispatcher hands ids to the 8 XCDs
@@ -1163,6 +1169,269 @@ __global__ __launch_bounds__(ap::NW * 64) __attribute__((amdgpu_waves_per_eu(1, 
   }
 }
 
+// Few queries a head (a decode step's one, a few speculated ones): the launch is bound by
+// streaming K and V once, which attention_fast_kernel, whose eight waves each compute 32
+// query slots of every key tile, does at 2 us per 64 keys and workgroup.  Here the four
+// waves of a workgroup share one block of 32 queries and take its 32-key tiles in turn, each
+// with two LDS stages of its own filled by DMA (buffer_load ... lds: 1 KiB of contiguous keys
+// per instruction) and no barrier in the loop; then the waves' (max, sum, O) states are
+// merged through LDS.  The keys of a block may be split over g.splits workgroups; each then
+// stores its merged state (fp32) to the workspace, and attention_merge_kernel joins them.
+// LDS tiles and fragments as in attention_pipe_kernel: K [key][DM] with 16-byte chunks
+// XOR-swizzled by key so that the 16 keys of a ds_read_b128 pass fall on 16 distinct bank
+// groups; V [key][DM] with 64-byte chunks XOR-swizzled so that the 4 keys of a transposing
+// read (ds_read_b64_tr_b16) do.  Scores, the lazily kept max and the rounding of P are
+// attention_fast_kernel's; row sums are of the unrounded p, in fp32.
+namespace ak {
+constexpr int NW = 4, BN = 32, BQ = 32;
+template <int DM>
+struct Geo {
+  static constexpr int ROW = DM * 2, CH = ROW / 16, TILE = BN * ROW, STAGE = 2 * TILE, WAVE = 2 * STAGE;
+  static constexpr int NI = TILE / 1024;  // DMA instructions per operand and tile
+  static constexpr int OROW = BQ + 1;     // merge area: O^T rows of 32 queries, padded
+  static constexpr int MERGE = DM * OROW * 4;
+  static constexpr int LDS = NW * (WAVE > MERGE ? WAVE : MERGE);
+};
+template <int DM>
+__device__ __forceinline__ int k_swz(int key) {
+  return DM == 128 ? key & 15 : (key >> 1) & 7;
+}
+template <int DM>
+__device__ __forceinline__ int v_swz(int key) {
+  return DM == 128 ? key & 3 : (key >> 1) & 1;
+}
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
+}
+}  // namespace ak
+
+template <typename T, int DM>
+__global__ __launch_bounds__(ak::NW * 64) void attention_keys_kernel(AttnArgs g) {
+  using G = ak::Geo<DM>;
+  typedef typename mfma_traits<T>::frag frag;
+  constexpr int DSUB = DM / 16, DBLK = DM / 32;
+  __shared__ __attribute__((aligned(1024))) char lds[G::LDS];
+  __shared__ float ml[ak::NW][2][ak::BQ];
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t lds_w = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds + wave * G::WAVE;
+  // Workgroup -> (head, split, query block): the query blocks of one head and split, which
+  // read the same keys, run next to one another on one XCD.
+  const int nq = g.q_blocks, groups = (int)(g.B * g.H) * g.splits;
+  int grp, qblk;
+  if (groups % 8 == 0) {
+    const int x = blockIdx.x % 8, local = blockIdx.x / 8;
+    grp = (local / nq) * 8 + x;
+    qblk = local % nq;
+  } else {
+    grp = blockIdx.x / nq;
+    qblk = blockIdx.x % nq;
+  }
+  const int bh = grp / g.splits, split = grp % g.splits;
+  const int b = bh / (int)g.H, h = bh % (int)g.H;
+  const int Sk = (int)g.Sk, Sq = (int)g.Sq, D = (int)g.D;
+  const int q0 = qblk * ak::BQ, qpos = q0 + (lane & 31);
+  int tiles = (Sk + ak::BN - 1) / ak::BN;
+  if (g.causal) tiles = min(tiles, qblk + 1);  // up to the tile of the block's last query
+  const int t0 = (int)((int64_t)tiles * split / g.splits), t1 = (int)((int64_t)tiles * (split + 1) / g.splits);
+  const int first = t0 + wave;
+  const int nt = first < t1 ? (t1 - first + ak::NW - 1) / ak::NW : 0;  // this wave's tiles: first + j NW
+
+  const uint16_t* Q = (const uint16_t*)g.q + b * g.qs[0] + h * g.qs[1];
+  u32x4 qraw[DSUB];
+#pragma unroll
+  for (int dd = 0; dd < DSUB; ++dd) {
+    qraw[dd] = u32x4{0u, 0u, 0u, 0u};
+    if (qpos < Sq && dd * 16 + half * 8 < D) qraw[dd] = *(const u32x4*)(Q + (int64_t)qpos * g.qs[2] + dd * 16 + half * 8);
+  }
+  // K and V resources end at the last key's D-th element (keys past Sk read zeros); K chunks
+  // past D are fetched from the end (zeros), V's reach only outputs past D.
+  const int ks2b = (int)g.ks[2] * 2, vs2b = (int)g.vs[2] * 2;
+  const uint32_t k_end = (uint32_t)((Sk - 1) * ks2b + D * 2);
+  const u32x4 rsK = ap::rsrc((const uint16_t*)g.k + b * g.ks[0] + h * g.ks[1], k_end);
+  const u32x4 rsV =
+      ap::rsrc((const uint16_t*)g.v + b * g.vs[0] + h * g.vs[1], (uint32_t)((Sk - 1) * vs2b + D * 2));
+  int vk[G::NI], vv[G::NI];
+#pragma unroll
+  for (int u = 0; u < G::NI; ++u) {
+    const int key = (u * 64 + lane) / G::CH, p = lane % G::CH;
+    const int kc = p ^ ak::k_swz<DM>(key);
+    vk[u] = kc * 8 < D ? key * ks2b + kc * 16 : 0x7fffffff;
+    vv[u] = key * vs2b + ((((p >> 2) ^ ak::v_swz<DM>(key)) << 2) | (p & 3)) * 16;
+  }
+  auto issue = [&](int j) {  // this wave's tile j into its stage j % 2: K, then V
+    const int key0 = (first + j * ak::NW) * ak::BN;
+    const uint32_t st = lds_w + (uint32_t)((j & 1) * G::STAGE);
+#pragma unroll
+    for (int u = 0; u < G::NI; ++u) ap::load_lds16(rsK, st + u * 1024, vk[u], key0 * ks2b);
+#pragma unroll
+    for (int u = 0; u < G::NI; ++u) ap::load_lds16(rsV, st + G::TILE + u * 1024, vv[u], key0 * vs2b);
+  };
+  if (nt > 0) issue(0);
+  if (nt > 1) issue(1);
+  frag qf[DSUB];
+#pragma unroll
+  for (int dd = 0; dd < DSUB; ++dd) {
+    uint16_t tmp[8];
+    const uint16_t* hv = (const uint16_t*)&qraw[dd];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) tmp[u] = elem<T>::from_float(elem<T>::to_float(hv[u]) * g.q_scale);
+    qf[dd] = __builtin_bit_cast(frag, *(const u32x4*)tmp);
+  }
+  int k_rd[DSUB], v_rd[DBLK];
+#pragma unroll
+  for (int dd = 0; dd < DSUB; ++dd)
+    k_rd[dd] = wave * G::WAVE + (lane & 31) * G::ROW + (((2 * dd + half) ^ ak::k_swz<DM>(lane & 31)) * 16);
+  {
+    const int gq = lane >> 4, r = (lane & 15) >> 2, q = lane & 3;
+#pragma unroll
+    for (int i = 0; i < DBLK; ++i)
+      v_rd[i] = wave * G::WAVE + G::TILE + (4 * (gq >> 1) + r) * G::ROW + ((i ^ ak::v_swz<DM>(r)) * 64) +
+                (16 * (gq & 1) + 4 * q) * 2;
+  }
+
+  floatx16 o[DBLK];
+#pragma unroll
+  for (int i = 0; i < DBLK; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
+  float m = -INFINITY, l = 0.f;  // l: this lane's half of the keys
+  for (int j = 0; j < nt; ++j) {
+    const int st = (j & 1) * G::STAGE;
+    const bool more = j + 1 < nt;
+    if (more)
+      ak::wait_vm<3 * G::NI>();
+    else
+      ak::wait_vm<G::NI>();
+    floatx16 s;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = 0.f;
+#pragma unroll
+    for (int dd = 0; dd < DSUB; ++dd) s = mfma_traits<T>::mma(*(const frag*)(lds + k_rd[dd] + st), qf[dd], s);
+    const int key0 = (first + j * ak::NW) * ak::BN;
+    if (key0 + ak::BN > Sk || (g.causal && key0 + ak::BN - 1 > q0)) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = key0 + acc_row(r, lane);
+        if (key >= Sk || (g.causal && qpos < key)) s[r] = -INFINITY;
+      }
+    }
+    float mx = s[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    const bool grow = mx > m + attn::RESCALE_LOG2;  // (true for the first tile: m is -inf)
+    if (__builtin_amdgcn_ballot_w64(grow)) {
+      const float m_new = grow ? mx : m;
+      const float alpha = grow ? __builtin_amdgcn_exp2f(m - m_new) : 1.0f;
+      l *= alpha;
+#pragma unroll
+      for (int i = 0; i < DBLK; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
+      m = m_new;
+    }
+    frag pf[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      u32x4 w;
+#pragma unroll
+      for (int sl = 0; sl < 4; ++sl) {
+        const float p0 = __builtin_amdgcn_exp2f(s[8 * t + 2 * sl] - m);
+        const float p1 = __builtin_amdgcn_exp2f(s[8 * t + 2 * sl + 1] - m);
+        l += p0 + p1;
+        w[sl] = attn::pack2<T>(p0, p1);
+      }
+      pf[t] = __builtin_bit_cast(frag, w);
+    }
+    if (more)
+      ak::wait_vm<2 * G::NI>();
+    else
+      ak::wait_vm<0>();
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < DBLK; ++i) {
+        const char* p = lds + v_rd[i] + st + t * (16 * G::ROW);
+        const ap::v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ap::v4i16*)p);
+        const ap::v4i16 hi =
+            __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) ap::v4i16*)(p + 8 * G::ROW));
+        const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+        o[i] = mfma_traits<T>::mma(__builtin_bit_cast(frag, u32x4{l2[0], l2[1], h2[0], h2[1]}), pf[t], o[i]);
+      }
+    // Every LDS read of this stage has returned before it is refilled.
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (j + 2 < nt) issue(j + 2);
+  }
+
+  // Merge the waves: O^T [d][query] and (m, l) per query through LDS.
+  l += __shfl_xor(l, 32, 64);
+  __syncthreads();  // other waves may still read their stages, which the merge area covers
+  float* mo = (float*)lds + wave * (DM * G::OROW);
+#pragma unroll
+  for (int i = 0; i < DBLK; ++i)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mo[(i * 32 + acc_row(r, lane)) * G::OROW + (lane & 31)] = o[i][r];
+  if (half == 0) {
+    ml[wave][0][lane] = m;
+    ml[wave][1][lane] = l;
+  }
+  __syncthreads();
+  const int rows = Sq - q0 < ak::BQ ? Sq - q0 : ak::BQ;
+  const float* all = (const float*)lds;
+  for (int e = tid; e < rows * DM; e += ak::NW * 64) {
+    const int q = e / DM, d = e % DM;
+    float mm = ml[0][0][q];
+#pragma unroll
+    for (int w = 1; w < ak::NW; ++w) mm = fmaxf(mm, ml[w][0][q]);
+    float acc = 0.f, sum = 0.f;
+#pragma unroll
+    for (int w = 0; w < ak::NW; ++w) {
+      const float mw = ml[w][0][q];
+      const float sc = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - mm);  // (a wave without tiles adds nothing)
+      sum += ml[w][1][q] * sc;
+      acc += all[w * (DM * G::OROW) + d * G::OROW + q] * sc;
+    }
+    if (g.splits == 1) {
+      if (d < D)
+        store_from_float(g.o, b * g.os[0] + h * g.os[1] + (int64_t)(q0 + q) * g.os[2] + d * g.os[3], g.o_dtype,
+                         acc / sum);
+    } else {
+      const int64_t row = ((int64_t)split * (g.B * g.H) + bh) * Sq + q0 + q;
+      g.part_o[row * DM + d] = acc;
+      if (d == 0) {
+        g.part_ml[row * 2] = mm;
+        g.part_ml[row * 2 + 1] = sum;
+      }
+    }
+  }
+}
+
+// Joins the splits of attention_keys_kernel: one wave per (head, query), lanes over d.
+template <int DM>
+__global__ __launch_bounds__(256) void attention_merge_kernel(AttnArgs g) {
+  const int lane = threadIdx.x & 63;
+  const int64_t rows = g.B * g.H * g.Sq, row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  float mm = -INFINITY;
+  for (int s = 0; s < g.splits; ++s) mm = fmaxf(mm, g.part_ml[(s * rows + row) * 2]);
+  float acc[DM / 64] = {}, sum = 0.f;
+  for (int s = 0; s < g.splits; ++s) {
+    const float ms = g.part_ml[(s * rows + row) * 2];
+    const float sc = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mm);  // (a split without tiles adds nothing)
+    sum += g.part_ml[(s * rows + row) * 2 + 1] * sc;
+#pragma unroll
+    for (int u = 0; u < DM / 64; ++u) acc[u] += g.part_o[(s * rows + row) * DM + u * 64 + lane] * sc;
+  }
+  const int64_t bh = row / g.Sq, q = row % g.Sq;
+#pragma unroll
+  for (int u = 0; u < DM / 64; ++u)
+    if (u * 64 + lane < g.D)
+      store_from_float(g.o, (bh / g.H) * g.os[0] + (bh % g.H) * g.os[1] + q * g.os[2] + (u * 64 + lane) * g.os[3],
+                       g.o_dtype, acc[u] / sum);
+}
+
 // Vector-load variant: two waves per SIMD (two workgroups per CU) so that one
 // workgroup's softmax and LDS traffic overlap the other's matrix work.
 template <typename T, int DM>
@@ -1179,7 +1448,7 @@ __global__ __launch_bounds__(AT_THREADS) void attention_generic_kernel(AttnArgs 
 // config: 0 = attention_fast_kernel where its conditions hold, else the four-wave kernels;
 // 1 = attention_pipe_kernel (head dim 128, the fast conditions); 2 = attention_fast_kernel
 // (the fast conditions); 3 = the four-wave kernels (attention_kernel, or
-// attention_generic_kernel for other strides).
+// attention_generic_kernel for other strides); 4 = attention_keys_kernel (the fast conditions).
 // A forced configuration whose conditions do not hold returns NT_ERR_INVALID unlaunched.
 // No keys: every query's weights are an empty softmax and its output is zero (as torch's
 // scaled_dot_product_attention defines it); o is filled, element by element over its strides.
@@ -1203,12 +1472,35 @@ static int attention_empty_keys(void* o, const int64_t* os, int o_dtype, int64_t
   return launch_status();
 }
 
+// attention_keys_kernel or attention_fast_kernel, measured fp16/bf16 with K and V rotated past
+// the caches.  A workgroup of the first takes 32 queries through 4,096 keys of D = 128 in about
+// 57 us, one of the second 256 queries in 107, so the first is the faster while one round of
+// its workgroups fits the chip or one block holds all the queries of a head (keys / fast us:
+// [8,32,1,4000,128] 93 / 150, [1,32,1,4096,128] 24 / 106, [4,32,64,4096,128] 57 / 108,
+// [32,32,32,4096,128] 369 / 441, [1,8,1024,1024,128] 17.4 / 32.6, [2,8,128,128,64] 6.2 / 12.7);
+// two blocks a head beat the four-wave kernel, too ([16,32,64,4096,128] 211 / 232).
+static bool attention_keys_wanted(int64_t BH, int64_t Sq) {
+  const int64_t nq = cdiv(Sq, ak::BQ);
+  return nq == 1 || nq * BH <= 256 || (nq == 2 && BH >= 512);
+}
+// Workgroups per query block: as many as fill the 256 CUs once, each with at least 32 tiles
+// (1,024 keys), at most 8: splits cost the merge launch (us at 1 / 2 / 4 / 8 / 16 splits:
+// [1,32,1,4096,128] 44 / 31 / 24 / 25 / 35; [4,32,1,4096,128] 54.6 / 52.8 / 55 / 62 / 82;
+// [1,8,4,8192,128] 60 / 37 / 25 / 20 / 22).
+static int attention_splits(int64_t BH, int64_t Sq, int64_t Sk) {
+  const int64_t blocks = cdiv(Sq, ak::BQ) * BH, tiles = cdiv(Sk, ak::BN);
+  return (int)std::max<int64_t>(1, std::min<int64_t>({256 / blocks, tiles / 32, 8}));
+}
+static int64_t attention_workspace(int64_t BH, int64_t Sq, int64_t Sk, int64_t D, int splits) {
+  return splits > 1 ? splits * BH * Sq * ((D <= 64 ? 64 : 128) + 2) * (int64_t)sizeof(float) : 0;
+}
+
 template <typename T>
 static int attention_launch(const void* q, const int64_t* qs, const void* k, const int64_t* ks, const void* v,
                             const int64_t* vs, void* o, const int64_t* os, int o_dtype, int64_t B, int64_t H,
                             int64_t Sq, int64_t Sk, int64_t D, float q_scale, int causal, hipStream_t stream,
-                            int config = 0) {
-  if (config < 0 || config > 3) return NT_ERR_INVALID;
+                            int config = 0, void* workspace = nullptr, int64_t workspace_bytes = 0) {
+  if (config < 0 || config > 4) return NT_ERR_INVALID;
   if (B < 0 || H < 0 || Sq < 0 || Sk < 0 || D < 0 || D > 128) return NT_ERR_INVALID;
   if (!valid_dtype(o_dtype)) return NT_ERR_INVALID;
   if (B * H * Sq * D == 0) return 0;
@@ -1253,7 +1545,30 @@ static int attention_launch(const void* q, const int64_t* qs, const void* k, con
   };
   const int64_t dm = D <= 64 ? 64 : 128;
   const bool fast_fits = fast_ok(dm), pipe_fits = D == 128 && fast_fits;
-  if ((config == 1 && !pipe_fits) || (config == 2 && !fast_fits)) return NT_ERR_INVALID;
+  const bool keys_fits = fast_fits && B * H <= 0x7fffffffLL / 64;
+  if ((config == 1 && !pipe_fits) || (config == 2 && !fast_fits) || (config == 4 && !keys_fits)) return NT_ERR_INVALID;
+  if (config == 4 || (config == 0 && keys_fits && attention_keys_wanted(B * H, Sq))) {
+    const int64_t qblocks = cdiv(Sq, ak::BQ);
+    // a causal block sees only the keys up to its queries: never split
+    int splits = config == 0 && !causal ? attention_splits(B * H, Sq, Sk) : 1;
+    if (splits > 1 && (!workspace || (uintptr_t)workspace % 16 || workspace_bytes < attention_workspace(B * H, Sq, Sk, D, splits)))
+      splits = 1;
+    if (qblocks * B * H * splits > 0x7fffffffLL) return NT_ERR_INVALID;
+    g.q_blocks = (int)qblocks;
+    g.splits = splits;
+    g.part_o = (float*)workspace;
+    g.part_ml = splits > 1 ? g.part_o + splits * B * H * Sq * dm : nullptr;
+    const dim3 gridK((unsigned)(qblocks * B * H * splits)), blkK(ak::NW * 64);
+    const dim3 gridM((unsigned)cdiv(B * H * Sq, 4));
+    if (dm == 64) {
+      hipLaunchKernelGGL((attention_keys_kernel<T, 64>), gridK, blkK, 0, stream, g);
+      if (splits > 1) hipLaunchKernelGGL((attention_merge_kernel<64>), gridM, dim3(256), 0, stream, g);
+    } else {
+      hipLaunchKernelGGL((attention_keys_kernel<T, 128>), gridK, blkK, 0, stream, g);
+      if (splits > 1) hipLaunchKernelGGL((attention_merge_kernel<128>), gridM, dim3(256), 0, stream, g);
+    }
+    return launch_status();
+  }
   // The eight-wave kernel is the default: measured on MI355X at B=4, H=32, S=4096, D=128
   // it runs 1,090-1,130 us non-causal against 1,140-1,270 us for the pipelined kernel.  Up
   // to 128 queries a head with at least 512 heads (B H), the four-wave kernel's 128-query
@@ -1488,4 +1803,17 @@ extern "C" int nt_attention_config_f16(NT_ATTN_PARAMS, int config) {
 }
 extern "C" int nt_attention_config_bf16(NT_ATTN_PARAMS, int config) {
   return nt::attention_launch<nt::bf16_t>(NT_ATTN_ARGS, config);
+}
+extern "C" int64_t nt_attention_workspace_size(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D, int causal,
+                                               int dtype) {
+  if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || D <= 0 || D > 128 || causal) return 0;
+  if (dtype != NT_DTYPE_F16 && dtype != NT_DTYPE_BF16) return 0;
+  if (!nt::attention_keys_wanted(B * H, Sq)) return 0;
+  return nt::attention_workspace(B * H, Sq, Sk, D, nt::attention_splits(B * H, Sq, Sk));
+}
+extern "C" int nt_attention_ws_f16(NT_ATTN_PARAMS, void* workspace, int64_t workspace_bytes) {
+  return nt::attention_launch<nt::f16_t>(NT_ATTN_ARGS, 0, workspace, workspace_bytes);
+}
+extern "C" int nt_attention_ws_bf16(NT_ATTN_PARAMS, void* workspace, int64_t workspace_bytes) {
+  return nt::attention_launch<nt::bf16_t>(NT_ATTN_ARGS, 0, workspace, workspace_bytes);
 }

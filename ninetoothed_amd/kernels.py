@@ -443,10 +443,12 @@ def conv2d(x, w, y, padding=(0, 0), stride=(1, 1), dilation=(1, 1), round_dtype=
 
 
 # ------------------------------------------------------------------- attention
-# Kernel configurations of the 16-bit attention that ``config`` can force (0: the eight-wave
-# kernel where its conditions hold): the one-wave-per-SIMD pipelined kernel (head dim 128),
-# the eight-wave kernel, the four-wave kernels (any strides).
-ATTENTION_CONFIGS = (1, 2, 3)
+# Kernel configurations of the 16-bit attention that ``config`` can force (0: the key-streaming
+# kernel for few queries or few heads, else the eight-wave kernel where its conditions hold):
+# the one-wave-per-SIMD pipelined kernel (head dim 128), the eight-wave kernel, the four-wave
+# kernels (any strides), the key-streaming kernel (whose keys config 0 may also split over
+# workgroups, through a workspace).
+ATTENTION_CONFIGS = (1, 2, 3, 4)
 
 
 def check_attention(q, k, v, o, config=0):
@@ -482,6 +484,24 @@ def bind_attention(q, k, v, o, causal=False, q_scale=LOG2E, config=0):
     qs, ks, vs, os_ = (_lib.int64_array(t.stride()) for t in (q, k, v, o))
     tail = (_lib.dtype_code(o.dtype), bsz, heads, sq, sk, d, float(q_scale), 1 if causal else 0)
     stream = _stream_of(device)
+    nbytes = 0
+    if not config and _lib.dtype_code(q.dtype) != _lib.DTYPE_F32:
+        nbytes = int(_lib.load().nt_attention_workspace_size(bsz, heads, sq, sk, d, 1 if causal else 0,
+                                                             _lib.dtype_code(q.dtype)))
+    if nbytes:
+        import torch
+
+        fn, name = _entry(f"nt_attention_ws_{_lib.dtype_suffix(q.dtype)}")
+
+        def launch(q, k, v, o):
+            # from torch's stream-ordered caching allocator on every call, as conv2d's
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+            code = fn(q.data_ptr(), qs, k.data_ptr(), ks, v.data_ptr(), vs, o.data_ptr(), os_, *tail, stream(),
+                      ws.data_ptr(), nbytes)
+            if code:
+                _raise(code, name)
+
+        return launch
 
     def launch(q, k, v, o):
         code = fn(q.data_ptr(), qs, k.data_ptr(), ks, v.data_ptr(), vs, o.data_ptr(), os_, *tail, stream(), *extra)

@@ -13,7 +13,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from ninetoothed_amd import kernels
+from ninetoothed_amd import _lib, kernels
 
 pytestmark = pytest.mark.gpu
 
@@ -1237,6 +1237,42 @@ def test_attention_pipe_bf16_against_eight_wave(causal):
     ref = _sdpa_ref(q, k, v, causal, scale)
     assert torch.allclose(o1.float(), ref, atol=2e-2, rtol=2e-2)
     assert torch.allclose(o1.float(), o2.float(), atol=2e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("b, h, sq, sk, d", (
+    (1, 1, 1, 1, 64), (1, 3, 1, 31, 128), (2, 4, 33, 33, 64), (1, 2, 4, 1000, 96), (1, 2, 1, 2047, 128),
+    (1, 3, 5, 4097, 64), (1, 8, 2, 9000, 128), (3, 16, 32, 1056, 40)))
+def test_attention_few_queries(b, h, sq, sk, d, dtype):
+    # The key-streaming kernel: forced, by default without a workspace (C ABI) and by default
+    # with one (its keys split over workgroups from 2,048 keys on), strided K and V, ragged
+    # key tiles, waves without a tile; scores that rise along the keys, so that every wave
+    # and split ends with a max of its own.
+    u = _randn((d,), torch.float32, 120) / math.sqrt(d)
+    q = (_randn((b, h, sq, d), torch.float32, 121) + 2.0 * u).to(dtype)
+    ramp = torch.linspace(0, 4, sk, device=DEV)[:, None] * u * math.sqrt(d)
+    kv = torch.empty((2, b, sk, h, d), dtype=dtype, device=DEV)
+    k, v = kv[0].transpose(1, 2), kv[1].transpose(1, 2)
+    k.copy_((_randn((b, h, sk, d), torch.float32, 122) + ramp).to(dtype))
+    v.copy_(_randn((b, h, sk, d), dtype, 123))
+    qs = kernels.LOG2E / math.sqrt(d)
+    tol = 1e-2 if dtype == torch.float16 else 2e-2
+    for causal in (False, True):
+        ref = _attention_ref64(q, k, v, causal, qs)
+        for config in (0, 4):
+            o = torch.full_like(q, 7.0)
+            kernels.attention(q, k, v, o, causal=causal, q_scale=qs, config=config)
+            assert torch.allclose(o.double(), ref, atol=tol, rtol=tol)
+    # with the workspace refused (too small), the same keys unsplit
+    lib, suffix = _lib.load(), _lib.dtype_suffix(dtype)
+    o = torch.full_like(q, 7.0)
+    strides = [_lib.int64_array(t.stride()) for t in (q, k, v, o)]
+    ws = torch.empty(16, dtype=torch.uint8, device=DEV)
+    code = getattr(lib, f"nt_attention_ws_{suffix}")(
+        q.data_ptr(), strides[0], k.data_ptr(), strides[1], v.data_ptr(), strides[2], o.data_ptr(), strides[3],
+        _lib.dtype_code(dtype), b, h, sq, sk, d, qs, 0, torch.cuda.current_stream().cuda_stream, ws.data_ptr(), 16)
+    assert code == 0
+    assert torch.allclose(o.double(), _attention_ref64(q, k, v, False, qs), atol=tol, rtol=tol)
 
 
 def test_attention_config_conditions_are_checked():
