@@ -288,7 +288,10 @@ int nt_conv2d_bf16(const void* x, const int64_t* x_strides, const void* w, const
  * 16-byte aligned rows, H W and C multiples of 8, C >= 96, a 16-bit y; H W no multiple of 8
  * through the workspace with rows padded to 8); 7 = the re-laid input through the DMA kernel
  * of 128 x 128 tiles (four waves, two workgroups per CU), as 1 otherwise; the default for
- * outputs of fewer than 136 tiles of 256 x 256).  A forced path whose
+ * outputs of fewer than 136 tiles of 256 x 256); 8 = the im2col matrix written out to the
+ * workspace and the filter, dense over (c, r, s), used in place, on the same kernel (C R S a
+ * multiple of 32; the default for small planes with no more output positions than output
+ * channels).  A forced path whose
  * conditions do not hold returns NT_ERR_INVALID before launching.  Replaces the
  * per-configuration launchers the reference's auto-tuner times
  * (src/ninetoothed/compiler/driver.py:975-1031, tests/test_conv2d.py:109-113). */

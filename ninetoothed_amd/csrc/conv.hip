@@ -14,6 +14,7 @@
 // MFMA-bound in principle (2 * N*P*Q * K * C*R*S flops per launch).
 #include "mfma_core.h"
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -1398,43 +1399,162 @@ __global__ __launch_bounds__(256) void rows_unpad_kernel(const uint16_t* __restr
   }
 }
 
-// Sum of conv_dma_kernel's split partials: one lane per 8 consecutive output positions of
-// one channel, rounded and stored as one 16-byte vector when they share an output row
-// (qvec), else element by element.
-template <typename T>
+// Sum of conv_dma_kernel's split partials: one lane per W consecutive output positions of one
+// channel.  W 8 (qvec): rounded and stored as one 16-byte vector, the positions sharing an
+// output row.  W 2: stored element by element; a small output's partials then come from four
+// times as many lanes (16 splits of [8,512,7,7] x 512, 12.8 MB: 10.2 -> 4.3 us).  Four
+// splits' loads are in flight at a time; the sum runs in the order of the splits.
+template <typename T, int W>
 __global__ __launch_bounds__(256) void conv_splitk_reduce_kernel(ConvArgs g) {
-  const int64_t mv = g.Mp / 8, total = g.K * mv;
+  typedef float vec_t __attribute__((ext_vector_type(W == 8 ? 4 : W)));
+  constexpr int NV = W == 8 ? 2 : 1, VE = W / NV;
+  const int64_t mv = g.Mp / W, total = g.K * mv;
   uint16_t* Y = (uint16_t*)g.y;
   for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < total; e += (int64_t)gridDim.x * 256) {
-    const int64_t k = e / mv, m = (e - k * mv) * 8;
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int sp = 0; sp < g.splits; ++sp) {
-      const float* src = g.part + ((int64_t)sp * g.K + k) * g.Mp + m;
-      const float4 a = *(const float4*)src, b = *(const float4*)(src + 4);
-      v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w;
-      v[4] += b.x; v[5] += b.y; v[6] += b.z; v[7] += b.w;
-    }
-    u32x4 ow;
+    const int64_t k = e / mv, m = (e - k * mv) * W;
+    float v[W];
 #pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      const float a = round_through(v[2 * d], g.round_dtype), b = round_through(v[2 * d + 1], g.round_dtype);
-      ow[d] = (uint32_t)elem<T>::from_float(a) | ((uint32_t)elem<T>::from_float(b) << 16);
+    for (int u = 0; u < W; ++u) v[u] = 0.f;
+    const float* src = g.part + k * g.Mp + m;
+    const int64_t step = g.K * g.Mp;
+    int sp = 0;
+    for (; sp + 4 <= g.splits; sp += 4) {
+      vec_t a[4][NV];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int h = 0; h < NV; ++h) a[i][h] = *(const vec_t*)(src + (sp + i) * step + h * VE);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int u = 0; u < W; ++u) v[u] += a[i][u / VE][u % VE];
     }
-    if (g.qvec) {
+    for (; sp < g.splits; ++sp)
+#pragma unroll
+      for (int h = 0; h < NV; ++h) {
+        const vec_t a = *(const vec_t*)(src + sp * step + h * VE);
+#pragma unroll
+        for (int u = 0; u < VE; ++u) v[h * VE + u] += a[u];
+      }
+    uint16_t o[W];
+#pragma unroll
+    for (int u = 0; u < W; ++u) o[u] = elem<T>::from_float(round_through(v[u], g.round_dtype));
+    if constexpr (W == 8) {
       const int64_t q = m % g.Q, t = m / g.Q;
       const int64_t p = t % g.P, n = t / g.P;
-      __builtin_nontemporal_store(ow, (u32x4*)(Y + n * g.ys[0] + k * g.ys[1] + p * g.ys[2] + q));
+      __builtin_nontemporal_store(*(const u32x4*)o, (u32x4*)(Y + n * g.ys[0] + k * g.ys[1] + p * g.ys[2] + q));
     } else {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < W; ++u) {
         const int64_t mu = m + u;
         if (mu < g.M) {
           const int64_t q = mu % g.Q, t = mu / g.Q;
-          Y[(t / g.P) * g.ys[0] + k * g.ys[1] + (t % g.P) * g.ys[2] + q * g.ys[3]] =
-              (uint16_t)(ow[u >> 1] >> (16 * (u & 1)));
+          Y[(t / g.P) * g.ys[0] + k * g.ys[1] + (t % g.P) * g.ys[2] + q * g.ys[3]] = o[u];
         }
       }
     }
+  }
+}
+
+// The im2col matrix [M = N P Q][C R S] (the reduction in the filter's own order c, r, s), for
+// filters large beside the output: a K-C-R-S filter dense over (c, r, s) is then used where it
+// lies, as the rows of a 1 x 1 filter over C R S channels, instead of being re-laid.  A
+// workgroup takes CB channels of one image: it stages their zero-padded planes in LDS, then
+// each lane writes one fixed 16-byte column chunk of rows m, m + RG, ... (its eight LDS
+// offsets computed once), so the lanes of a row write CB R S contiguous elements.
+constexpr int PLANES_LDS = 60 * 1024;
+// Zero-padded planes [CB][Hp][Wp] of channels c0 .. c0 + CB - 1 of one image into LDS (zeros past
+// channel Cr); eight loads per lane in flight (one at a time, the launch was a chain of memory
+// latencies).  Divisions by multiplication: exact for element numbers below 2^15.
+__device__ __forceinline__ void stage_planes(const uint16_t* X, const ConvArgs& g, int c0, int CB, int Hp, int Wp,
+                                             uint16_t* plane) {
+  const int HWp = Hp * Wp, total = CB * HWp, ph = (int)g.ph, pw = (int)g.pw, H = (int)g.H, W = (int)g.W;
+  const int cr = (int)g.Cr - c0;
+  const uint32_t mhw = HWp > 1 ? (uint32_t)(0xffffffffu / (uint32_t)HWp + 1) : 0u;
+  const uint32_t mw = Wp > 1 ? (uint32_t)(0xffffffffu / (uint32_t)Wp + 1) : 0u;
+  constexpr int U = 8;
+  for (int e0 = threadIdx.x; e0 < total; e0 += 256 * U) {
+    uint16_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int e = e0 + u * 256;
+      const int c = mhw ? (int)__umulhi((uint32_t)e, mhw) : e, t = e - c * HWp;
+      const int hp = mw ? (int)__umulhi((uint32_t)t, mw) : t, h = hp - ph, w = t - hp * Wp - pw;
+      const bool ok = e < total && c < cr && (uint32_t)h < (uint32_t)H && (uint32_t)w < (uint32_t)W;
+      v[u] = ok ? X[c * g.xs[1] + h * g.xs[2] + w * g.xs[3]] : (uint16_t)0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (e0 + u * 256 < total) plane[e0 + u * 256] = v[u];
+  }
+}
+
+__global__ __launch_bounds__(256) void conv_cols_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ cols,
+                                                        ConvArgs g, int CB, int Hp, int Wp) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t plane[];
+  const int tid = threadIdx.x, cblocks = (int)g.C / CB;
+  const int n = blockIdx.x / cblocks, c0 = (blockIdx.x % cblocks) * CB;
+  stage_planes(x + (int64_t)n * g.xs[0] + (int64_t)c0 * g.xs[1], g, c0, CB, Hp, Wp, plane);
+  const int HWp = Hp * Wp;
+  const int RS = (int)(g.R * g.S), S = (int)g.S, J = CB * RS / 8, RG = 256 / J;
+  const int j = tid % J, r0 = tid / J;
+  int off[8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u) {
+    const int kk = j * 8 + u, c = kk / RS, rs = kk - c * RS, r = rs / S, s = rs - r * S;
+    off[u] = c * HWp + r * (int)g.dh * Wp + s * (int)g.dw;
+  }
+  __syncthreads();
+  if (r0 >= RG) return;
+  const int Q = (int)g.Q, PQ = (int)g.P * Q;
+  uint16_t* out = cols + ((int64_t)n * PQ) * g.KG + (int64_t)c0 * RS + j * 8;
+  for (int m = r0; m < PQ; m += RG) {
+    const int p = m / Q, q = m - p * Q;
+    const uint16_t* base = plane + p * (int)g.sh * Wp + q * (int)g.sw;
+    u32x4 v;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) v[d] = (uint32_t)base[off[2 * d]] | ((uint32_t)base[off[2 * d + 1]] << 16);
+    *(u32x4*)(out + m * g.KG) = v;
+  }
+}
+
+// Both re-layouts in one launch for small planes of any width and strides, where
+// nchw_to_nhwc_pad_kernel's 64-position rows are mostly padding: workgroups [0, in_blocks) take
+// CB channels (32 or 64) of one image, staged as whole zero-padded planes in LDS and written as
+// 16-byte runs of 8 channels; the others transpose a contiguous 3 x 3 filter as
+// filter_cb9_kernel does, seven 32-channel units each (units 0: the filter is re-laid apart).
+__global__ __launch_bounds__(256) void conv_planes_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ xp,
+                                                          const uint16_t* __restrict__ w, uint16_t* __restrict__ wt,
+                                                          ConvArgs g, int CB, int Hp, int Wp, int in_blocks, int units) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t plane[];
+  const int tid = threadIdx.x;
+  if ((int)blockIdx.x >= in_blocks) {
+    constexpr int U = 7, CH = 36;
+    const int u0 = ((int)blockIdx.x - in_blocks) * U;
+    const int n = (units - u0 < U ? units - u0 : U) * CH;
+    if (tid < n) *(u32x4*)(plane + tid * 8) = *(const u32x4*)(w + (int64_t)u0 * 288 + tid * 8);
+    __syncthreads();
+    if (tid < n) {
+      const int un = tid / CH, q = tid - un * CH, rs = q >> 2, c8 = (q & 3) * 8;
+      uint16_t v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = plane[un * 288 + (c8 + i) * 9 + rs];
+      *(u32x4*)(wt + (int64_t)u0 * 288 + tid * 8) = *(const u32x4*)v;
+    }
+    return;
+  }
+  const int cblocks = (int)g.C / CB;
+  const int n = blockIdx.x / cblocks, c0 = (blockIdx.x % cblocks) * CB, HWp = Hp * Wp;
+  stage_planes(x + (int64_t)n * g.xs[0] + (int64_t)c0 * g.xs[1], g, c0, CB, Hp, Wp, plane);
+  __syncthreads();
+  const int lg = CB == 64 ? 3 : 2;  // 8-channel chunks per position
+  uint16_t* out = xp + (int64_t)n * HWp * g.C + c0;
+  for (int e = tid; e < HWp << lg; e += 256) {
+    const int pos = e >> lg, c8 = (e & ((1 << lg) - 1)) * 8;
+    uint16_t v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = plane[(c8 + u) * HWp + pos];
+    *(u32x4*)(out + (int64_t)pos * g.C + c8) = *(const u32x4*)v;
   }
 }
 
@@ -1481,6 +1601,44 @@ static int64_t conv_splits(int64_t tiles, int64_t nk, int64_t K, int64_t M, int6
   return 1;
 }
 
+// The im2col path by default: no more output positions than output channels, so that the
+// matrix is no larger than the filter whose re-layout it saves, and small planes.  fp16 us,
+// im2col / re-laid with conv_planes_kernel (or conv_relayout_pipe_kernel for 16 x 16):
+// [8,512,7,7] x 512 26.3 / 28.1, [2,512,14,14] x 512 29.2 / 30.9, [1,1280,16,16] x 1280 42 / 68,
+// [2,1280,16,16] x 1280 61 / 83, [1,512,7,7] x 512 19.8 / 19.5, [1,256,14,14] x 256 19.9 / 19.7;
+// with more positions [32,512,7,7] x 512 40.3 / 37.8, [32,256,14,14] x 256 44.5 / 41.1.
+// Larger planes stage slowly (LDS leaves one workgroup a CU): [1,512,28,28] x 512 42.8 against
+// 36.1 on nchw_to_nhwc_pad_kernel, [4,128,28,28] x 128 40.6 / 29.8.
+constexpr int64_t PLANES_BELOW = 400;  // padded positions of a plane
+static bool cols_wanted(int64_t M, int64_t K, int64_t R, int64_t S, int64_t Hp, int64_t Wp) {
+  return R * S > 1 && M <= K && Hp * Wp < PLANES_BELOW;
+}
+
+// Bytes of the im2col path's split partials when nothing limits the splits.
+static int64_t cols_partials(int64_t K, int64_t KG, int64_t M) {
+  const int64_t Mp = cdiv(M, 8) * 8;
+  int64_t per = 0;
+  const int64_t sp = conv_splits(cdiv(K, 128) * cdiv(M, 128), KG / 32, K, Mp, INT64_MAX, &per);
+  return sp > 1 ? sp * K * Mp * 4 : 0;
+}
+
+template <typename T>
+static void conv_reduce_launch(const ConvArgs& g, hipStream_t stream) {
+  const int64_t blocks = cdiv(g.K * (g.Mp / (g.qvec ? 8 : 2)), 256);
+  const dim3 grid((unsigned)(blocks < 4096 ? blocks : 4096));
+  if (g.qvec)
+    hipLaunchKernelGGL((conv_splitk_reduce_kernel<T, 8>), grid, dim3(256), 0, stream, g);
+  else
+    hipLaunchKernelGGL((conv_splitk_reduce_kernel<T, 2>), grid, dim3(256), 0, stream, g);
+}
+
+// Channels per workgroup of conv_cols_kernel (0: its LDS planes or lanes do not fit).
+static int64_t cols_channels(int64_t C, int64_t Hp, int64_t Wp, int64_t RS) {
+  for (int64_t cb : {16, 8})
+    if (C % cb == 0 && cb * Hp * Wp * 2 <= PLANES_LDS && cb * RS / 8 <= 256) return cb;
+  return 0;
+}
+
 template <typename T>
 static int conv_launch(const void* x, const int64_t* xs, const void* w, const int64_t* ws, void* y, const int64_t* ys,
                        int y_dtype, int64_t N, int64_t C, int64_t H, int64_t W, int64_t K, int64_t R, int64_t S,
@@ -1492,9 +1650,10 @@ static int conv_launch(const void* x, const int64_t* xs, const void* w, const in
   // workspace), 4 = re-laid input through the DMA kernel of 224-position tiles, 5 = the
   // input read in place by conv_strip224_kernel (only the filter re-laid), 6 = 1 x 1 filters
   // as a batch of products on gemm_dma128_kernel, 7 = re-laid input through the DMA kernel
-  // of 128 x 128 tiles.  A forced path whose conditions do not hold is rejected before
-  // launching.
-  if (config < 0 || config > 7) return NT_ERR_INVALID;
+  // of 128 x 128 tiles, 8 = the im2col matrix written out (conv_cols_kernel) and the filter in
+  // place, on the 128 x 128-tile kernel.  A forced path whose conditions do not hold is rejected
+  // before launching.
+  if (config < 0 || config > 8) return NT_ERR_INVALID;
   if (N < 0 || C < 0 || H < 0 || W < 0 || K < 0 || R < 0 || S < 0 || P < 0 || Q < 0 || ph < 0 || pw < 0 || sh <= 0 ||
       sw <= 0 || dh <= 0 || dw <= 0)
     return NT_ERR_INVALID;
@@ -1573,6 +1732,45 @@ static int conv_launch(const void* x, const int64_t* xs, const void* w, const in
   // Its output as 16-byte runs of 8 positions of one channel, or else element by element.
   g.qvec = Q % 8 == 0 && ys[3] == 1 && ys[0] % 8 == 0 && ys[1] % 8 == 0 && ys[2] % 8 == 0 && (uintptr_t)y % 16 == 0;
   g.Mp = cdiv(g.M, 8) * 8;
+  // The im2col path: a filter dense over (c, r, s) in place, whole 32-deep k-tiles, the matrix
+  // and the split partials in the workspace.
+  if (config == 8 || (config == 0 && cols_wanted(g.M, K, R, S, Hp, Wp))) {
+    const int64_t KG = C * R * S, cb = cols_channels(C, Hp, Wp, R * S);
+    const int64_t cols_bytes = cdiv(g.M * KG * 2, 256) * 256;
+    const bool fits = cb > 0 && R * S > 0 && KG >= 96 && KG % 32 == 0 && ws[3] == 1 && ws[2] == S && ws[1] == R * S &&
+                      ws[0] == KG && (uintptr_t)w % 16 == 0 && y_dtype == elem<T>::code && g.M * KG * 2 < 0x7fffffffLL &&
+                      K * KG * 2 < 0x7fffffffLL && workspace != nullptr && (uintptr_t)workspace % 256 == 0 &&
+                      workspace_bytes >= cols_bytes + (config == 0 ? cols_partials(K, KG, g.M) : 0) &&
+                      N * (C / cb) <= 0x7fffffffLL &&
+                      (P - 1) * sh + (R - 1) * dh < Hp && (Q - 1) * sw + (S - 1) * dw < Wp;
+    if (config == 8 && !fits) return NT_ERR_INVALID;
+    if (fits) {
+      uint16_t* cols = (uint16_t*)workspace;
+      hipLaunchKernelGGL(conv_cols_kernel, dim3((unsigned)(N * (C / cb))), dim3(256), (size_t)(cb * Hp * Wp * 2), stream,
+                         (const uint16_t*)x, cols, g, (int)cb, (int)Hp, (int)Wp);
+      // the product as a 1 x 1 convolution of a P x Q image of KG channels
+      g.C = KG;
+      g.R = g.S = 1;
+      g.H = P;
+      g.W = Q;
+      g.ph = g.pw = 0;
+      g.sh = g.sw = g.dh = g.dw = 1;
+      g.cb_order = 1;
+      g.tiles_k = (int)cdiv(K, 128);
+      g.tiles_m = (int)cdiv(g.M, 128);
+      const int64_t tiles = (int64_t)g.tiles_k * g.tiles_m;
+      int64_t per = KG / 32;
+      const int64_t sp = conv_splits(tiles, KG / 32, K, g.Mp, workspace_bytes - cols_bytes, &per);
+      if (sp * tiles > 0x7fffffffLL) return NT_ERR_INVALID;
+      g.splits = (int)sp;
+      g.kt_per = (int)per;
+      g.part = sp > 1 ? (float*)((char*)workspace + cols_bytes) : nullptr;
+      hipLaunchKernelGGL((conv_dma_kernel<T, 128>), dim3((unsigned)(sp * tiles)), dim3(256), 0, stream,
+                         (const uint16_t*)cols, (const uint16_t*)w, g, P, Q);
+      if (sp > 1) conv_reduce_launch<T>(g, stream);
+      return launch_status();
+    }
+  }
   // conv_strip224_kernel: a 3 x 3 filter, whole output rows per 224-position tile (Q divides
   // 224, the tile's TR rows divide P), stride and dilation 1, 32-channel blocks, input rows of
   // unit w stride in 16-byte chunks (W % 8 == 0, 16-byte aligned), a strip row of Q + 16
@@ -1677,12 +1875,29 @@ static int conv_launch(const void* x, const int64_t* xs, const void* w, const in
         hipLaunchKernelGGL((conv_relayout_kernel<T, false>), dim3((unsigned)(N * Hp + fblocks)), dim3(256), 0, stream,
                            (const uint16_t*)x, xp, (const uint16_t*)w, wt, g, Hp, Wp);
     } else {
-      const int64_t relayout_blocks = N * Hp * cdiv(Cl, 64);
-      if (relayout_blocks > 0x7fffffffLL) return NT_ERR_INVALID;
-      hipLaunchKernelGGL(nchw_to_nhwc_pad_kernel<T>, dim3((unsigned)relayout_blocks), dim3(256), 0, stream,
-                         (const uint16_t*)x, xp, g, Hp, Wp);
-      hipLaunchKernelGGL(filter_krsc_kernel<T>, dim3((unsigned)fblocks), dim3(256), 0, stream, (const uint16_t*)w, wt,
-                         g);
+      // small planes: 64 channels per workgroup when that still gives every CU one, else 32
+      const int64_t cbp = Cl % 64 == 0 && N * (Cl / 64) >= 256 && 64 * Hp * Wp * 2 <= PLANES_LDS ? 64 : 32;
+      const bool planes = Hp * Wp < PLANES_BELOW && cbp * Hp * Wp * 2 <= PLANES_LDS && N * (Cl / cbp) <= 0x3fffffff;
+      const bool filter9 = dma && R == 3 && S == 3 && Cl == C && ws[3] == 1 && ws[2] == 3 && ws[1] == 9 &&
+                           ws[0] == C * 9 && (uintptr_t)w % 16 == 0 && K * (C / 32) <= 0x3fffffff;
+      if (planes) {
+        const int64_t in_blocks = N * (Cl / cbp), units = filter9 ? K * (C / 32) : 0;
+        const int64_t lds = std::max<int64_t>(cbp * Hp * Wp * 2, 7 * 288 * 2);
+        hipLaunchKernelGGL(conv_planes_kernel, dim3((unsigned)(in_blocks + cdiv(units, 7))), dim3(256), (size_t)lds, stream,
+                           (const uint16_t*)x, xp, (const uint16_t*)w, wt, g, (int)cbp, (int)Hp, (int)Wp,
+                           (int)in_blocks, (int)units);
+      } else {
+        const int64_t relayout_blocks = N * Hp * cdiv(Cl, 64);
+        if (relayout_blocks > 0x7fffffffLL) return NT_ERR_INVALID;
+        hipLaunchKernelGGL(nchw_to_nhwc_pad_kernel<T>, dim3((unsigned)relayout_blocks), dim3(256), 0, stream,
+                           (const uint16_t*)x, xp, g, Hp, Wp);
+      }
+      if (!planes && filter9)
+        hipLaunchKernelGGL(filter_cb9_kernel, dim3((unsigned)cdiv(K * (C / 32), 4)), dim3(144), 0, stream,
+                           (const uint16_t*)w, wt, (int)(K * (C / 32)));
+      else if (!filter9)
+        hipLaunchKernelGGL(filter_krsc_kernel<T>, dim3((unsigned)fblocks), dim3(256), 0, stream, (const uint16_t*)w,
+                           wt, g);
     }
     if (m224) {
       g.tiles_m = (int)tiles_m224;
@@ -1698,11 +1913,7 @@ static int conv_launch(const void* x, const int64_t* xs, const void* w, const in
       else
         hipLaunchKernelGGL(conv_dma_kernel<T>, dim3((unsigned)(sp * tk * tm)), dim3(512), 0, stream,
                            (const uint16_t*)xp, (const uint16_t*)wt, g, Hp, Wp);
-      if (sp > 1) {
-        const int64_t vecs = K * (g.Mp / 8);
-        hipLaunchKernelGGL(conv_splitk_reduce_kernel<T>, dim3((unsigned)(cdiv(vecs, 256) < 4096 ? cdiv(vecs, 256) : 4096)),
-                           dim3(256), 0, stream, g);
-      }
+      if (sp > 1) conv_reduce_launch<T>(g, stream);
     } else
       hipLaunchKernelGGL(conv_nhwc_kernel<T>, dim3((unsigned)(tiles_k * tiles_m)), dim3(512), 0, stream,
                          (const uint16_t*)xp, (const uint16_t*)wt, g, Hp, Wp);
@@ -1720,8 +1931,9 @@ static int conv_launch(const void* x, const int64_t* xs, const void* w, const in
 
 }  // namespace nt
 
-extern "C" int64_t nt_conv2d_workspace_size(int64_t N, int64_t C, int64_t H, int64_t W, int64_t K, int64_t R,
-                                            int64_t S, int64_t ph, int64_t pw, int dtype) {
+// The re-laid path's workspace: what conv2d always took.
+static int64_t conv_relaid_workspace(int64_t N, int64_t C, int64_t H, int64_t W, int64_t K, int64_t R, int64_t S,
+                                     int64_t ph, int64_t pw, int dtype) {
   if (N <= 0 || C <= 0 || H <= 0 || W <= 0 || K <= 0 || R <= 0 || S <= 0 || ph < 0 || pw < 0) return 0;
   if (dtype != NT_DTYPE_F16 && dtype != NT_DTYPE_BF16) return 0;
   // Enough for either layout's channels (rounded up to 64, or the DMA kernel's), plus the
@@ -1735,6 +1947,17 @@ extern "C" int64_t nt_conv2d_workspace_size(int64_t N, int64_t C, int64_t H, int
   const int64_t sp = nt::conv_splits(nt::cdiv(K, nt::CB_K) * nt::cdiv(M, nt::CB_M), cd * R * S / 32, K, M, INT64_MAX,
                                      &per);
   return base + (sp > 1 ? sp * K * M * 4 : 0);
+}
+
+extern "C" int64_t nt_conv2d_workspace_size(int64_t N, int64_t C, int64_t H, int64_t W, int64_t K, int64_t R,
+                                            int64_t S, int64_t ph, int64_t pw, int dtype) {
+  const int64_t base = conv_relaid_workspace(N, C, H, W, K, R, S, ph, pw, dtype);
+  const int64_t P = H + 2 * ph - R + 1, Q = W + 2 * pw - S + 1;
+  // The im2col matrix and its split partials, where that path is the default at stride 1 (a
+  // larger stride has fewer positions).
+  if (base == 0 || P <= 0 || Q <= 0 || !nt::cols_wanted(N * P * Q, K, R, S, H + 2 * ph, W + 2 * pw)) return base;
+  const int64_t KG = C * R * S;
+  return std::max(base, nt::cdiv(N * P * Q * KG * 2, 256) * 256 + nt::cols_partials(K, KG, N * P * Q));
 }
 
 #define NT_CONV_ENTRY(NAME, T)                                                                                       \
@@ -1798,7 +2021,8 @@ int current_scratch(void** out) {
                       int y_dtype, int64_t N, int64_t C, int64_t H, int64_t W, int64_t K, int64_t R, int64_t S,       \
                       int64_t P, int64_t Q, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh, int64_t dw,   \
                       int round_dtype, hipStream_t stream) {                                                          \
-    if (nt_conv2d_workspace_size(N, C, H, W, K, R, S, ph, pw, CODE) > NT_CONV2D_SCRATCH_BYTES) return NT_ERR_SCRATCH; \
+    /* (a larger im2col matrix leaves the call on the re-laid path) */                                               \
+    if (conv_relaid_workspace(N, C, H, W, K, R, S, ph, pw, CODE) > NT_CONV2D_SCRATCH_BYTES) return NT_ERR_SCRATCH;    \
     void* ws_ptr = nullptr;                                                                                          \
     if (int e = current_scratch(&ws_ptr)) return e;                                                                  \
     return nt::conv_launch<T>(x, xs, w, ws, y, ys, y_dtype, N, C, H, W, K, R, S, P, Q, ph, pw, sh, sw, dh, dw,       \

@@ -953,6 +953,31 @@ def test_conv2d_strip224_rejects_unfit_calls():
     call(None, (32, 3, 3), x=xt)
 
 
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("case", (  # n, c, h, w, k, r, s, padding, stride, dilation
+    (1, 32, 7, 7, 64, 3, 3, (1, 1), (1, 1), (1, 1)), (3, 64, 13, 11, 520, 3, 3, (1, 0), (1, 1), (1, 1)),
+    (2, 96, 14, 14, 40, 3, 3, (1, 1), (2, 2), (1, 1)), (2, 160, 9, 17, 264, 3, 3, (2, 2), (1, 2), (2, 2)),
+    (1, 32, 17, 17, 300, 2, 2, (0, 0), (1, 1), (1, 1)), (5, 8, 6, 5, 200, 4, 4, (3, 2), (1, 1), (1, 1)),
+    (1, 1280, 8, 8, 320, 3, 3, (1, 1), (1, 1), (1, 1)), (2, 48, 18, 18, 33, 5, 5, (1, 1), (1, 1), (1, 1))))
+def test_conv2d_small_planes(case, dtype):
+    # Small planes: the im2col matrix with the filter in place (configuration 8, where C R S is a
+    # multiple of 32) and the plane re-layout (configuration 7), by default and forced, on a
+    # contiguous input and on channels-last strides; partial channel blocks and tiles, splits.
+    n, c, h, w_, k, r, s, pad, stride, dil = case
+    x = _randn((n, c, h, w_), dtype, 130)
+    w = _randn((k, c, r, s), dtype, 131, 1.0 / math.sqrt(c * r * s))
+    ref = F.conv2d(x.double().cpu(), w.double().cpu(), padding=pad, stride=stride, dilation=dil)
+    ws = torch.empty(1 << 26, dtype=torch.uint8, device=DEV)
+    tol = 2e-2 if dtype == torch.bfloat16 else 4e-3  # the result's rounding at magnitudes up to about 4
+    configs = (0, 7) + ((8,) if c * r * s % 32 == 0 else ())
+    for config in configs:
+        for xv in (x, x.contiguous(memory_format=torch.channels_last)):
+            y = torch.full(ref.shape, 7.0, dtype=dtype, device=DEV)
+            ws.fill_(0xff)  # stale workspace contents (NaN patterns) must not reach the result
+            kernels.conv2d(xv, w, y, padding=pad, stride=stride, dilation=dil, workspace=ws, config=config)
+            assert torch.allclose(y.double().cpu(), ref, atol=tol, rtol=tol)
+
+
 @pytest.mark.parametrize("flip", ("w", "h"))
 @pytest.mark.parametrize("config", (0, 1, 3, 4, 7))
 @pytest.mark.parametrize("xshape", ((4, 64, 15, 13), (17, 64, 45, 45)))
