@@ -378,9 +378,10 @@ def conv2d_workspace_bytes(x, w, padding=(0, 0)):
 # the direct kernel (no workspace), re-laid input through the DMA kernel of 224-position
 # tiles, the input read in place by the 224-position strip kernel (only the filter re-laid),
 # 1 x 1 filters as a batch of products on the 128 x 128-tile GEMM kernel, re-laid input
-# through the DMA kernel of 128 x 128 tiles, the im2col matrix written out and the filter in
-# place.
-CONV_CONFIGS = (1, 2, 3, 4, 5, 6, 7, 8)
+# through the DMA kernel of 128 x 128 tiles.  CONV_FORCED adds the im2col matrix written out
+# with the filter in place, which config 0 takes for small planes and the tuner does not time.
+CONV_CONFIGS = (1, 2, 3, 4, 5, 6, 7)
+CONV_FORCED = CONV_CONFIGS + (8,)
 
 
 def check_conv2d(x, w, y, round_dtype=None, config=0):
@@ -395,8 +396,8 @@ def check_conv2d(x, w, y, round_dtype=None, config=0):
         raise ValueError("conv2d shape mismatch")
     _lib.dtype_code(y.dtype)
     rd = _lib.DTYPE_NONE if round_dtype is None else _lib.dtype_code(round_dtype)
-    if config and config not in CONV_CONFIGS:
-        raise TypeError(f"conv2d config {config} is not one of {CONV_CONFIGS}")
+    if config and config not in CONV_FORCED:
+        raise TypeError(f"conv2d config {config} is not one of {CONV_FORCED}")
     return _entry_name("nt_conv2d_config" if config else "nt_conv2d", x.dtype), rd
 
 
@@ -447,9 +448,10 @@ def conv2d(x, w, y, padding=(0, 0), stride=(1, 1), dilation=(1, 1), round_dtype=
 # Kernel configurations of the 16-bit attention that ``config`` can force (0: the key-streaming
 # kernel for few queries or few heads, else the eight-wave kernel where its conditions hold):
 # the one-wave-per-SIMD pipelined kernel (head dim 128), the eight-wave kernel, the four-wave
-# kernels (any strides), the key-streaming kernel (whose keys config 0 may also split over
-# workgroups, through a workspace).
-ATTENTION_CONFIGS = (1, 2, 3, 4)
+# kernels (any strides).  ATTENTION_FORCED adds the key-streaming kernel (whose keys config 0
+# may also split over workgroups, through a workspace), which the tuner does not time.
+ATTENTION_CONFIGS = (1, 2, 3)
+ATTENTION_FORCED = ATTENTION_CONFIGS + (4,)
 
 
 def check_attention(q, k, v, o, config=0):
@@ -465,8 +467,8 @@ def check_attention(q, k, v, o, config=0):
         raise ValueError("attention head dim must be <= 128")
     _lib.dtype_code(o.dtype)
     if config:
-        if config not in ATTENTION_CONFIGS or _lib.dtype_suffix(q.dtype) not in ("f16", "bf16"):
-            raise TypeError(f"attention config {config} needs fp16/bf16 operands and one of {ATTENTION_CONFIGS}")
+        if config not in ATTENTION_FORCED or _lib.dtype_suffix(q.dtype) not in ("f16", "bf16"):
+            raise TypeError(f"attention config {config} needs fp16/bf16 operands and one of {ATTENTION_FORCED}")
         return _entry_name("nt_attention_config", q.dtype)
     return _entry_name("nt_attention", q.dtype)
 
