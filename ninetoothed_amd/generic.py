@@ -41,6 +41,7 @@ import copy
 import ctypes
 import dataclasses
 import hashlib
+import re
 import threading
 
 import numpy as np
@@ -85,7 +86,21 @@ _STORAGE = {
     "bool": ("bool", "bool", "{}", "{}"),
 }
 
+_SIZES = {"float8_e4m3fn": 1, "float8_e5m2": 1, "float16": 2, "bfloat16": 2, "float32": 4, "float64": 8, "int8": 1,
+          "uint8": 1, "int16": 2, "int32": 4, "int64": 8, "bool": 1}
+
 _PRELUDE = r"""
+// N consecutive elements, loaded and stored together wherever they start (16-byte global
+// accesses need no more than the element's alignment here).
+template <typename T, int N> struct nt_vec { T e[N]; };
+template <int N, typename T> __device__ __forceinline__ nt_vec<T, N> nt_ldv(const T* p) {
+  nt_vec<T, N> v;
+  __builtin_memcpy(&v, p, sizeof(v));
+  return v;
+}
+template <int N, typename T> __device__ __forceinline__ void nt_stv(T* p, const nt_vec<T, N>& v) {
+  __builtin_memcpy(p, &v, sizeof(v));
+}
 __device__ __forceinline__ float ld_f16(unsigned short b) { return (float)__builtin_bit_cast(_Float16, b); }
 __device__ __forceinline__ unsigned short st_f16(float x) { return __builtin_bit_cast(unsigned short, (_Float16)x); }
 __device__ __forceinline__ float r_f16(float x) { return (float)(_Float16)x; }
@@ -871,16 +886,21 @@ def _shapes(ctx, values, const_value, carried=None):
 def _unravel(idx, shape):
     """C expressions of the coordinates of row-major element ``idx`` of ``shape``."""
     coords, stride = [], 1
-    for size in reversed(shape):
+    outermost = next((i for i, size in enumerate(shape) if size != 1), None)  # idx is below the product: no modulo
+    for axis, size in reversed(tuple(enumerate(shape))):
         if size == 1:
             coords.append("0")
         else:
-            coords.append(f"(({idx} / {stride}LL) % {size}LL)" if stride > 1 else f"({idx} % {size}LL)")
+            q = f"({idx} / {stride}LL)" if stride > 1 else f"{idx}"
+            coords.append(q if axis == outermost else f"({q} % {size}LL)")
         stride *= size
     return tuple(reversed(coords))
 
 
 def _ravel(coords, shape):
+    for var in ("j", "l"):  # an index just unravelled over this shape
+        if coords == _unravel(var, shape) and coords.count("0") != len(coords):
+            return var
     terms, stride = [], 1
     for c, size in zip(reversed(coords), reversed(shape)):
         if size != 1:
@@ -898,6 +918,7 @@ class _TileEmitter(_Emitter):
         self.plan = plan
         self.types = plan.types
         self.shapes = plan.shapes
+        self.vec = 0  # elements per vector of the loop being emitted (0: element by element)
 
     def context(self, root, coords, tag, more=()):
         """Lines computing ``root`` at ``coords`` (and each (value, coords) of ``more``)."""
@@ -910,6 +931,28 @@ class _TileEmitter(_Emitter):
             if id(v) in self.coords:
                 self.emit(v)
         return self.lines
+
+    def vector_start(self, name, ks, lin):
+        """C element number at which the vector of this load starts, where the current loop
+        (``self.vec`` consecutive values of ``self.var`` per step, the first ``self.var`` + "0")
+        reads consecutive elements of ``name``; None otherwise."""
+        if not self.vec or ks or self.plan.forms.get(name, (0, None))[0] != 1:
+            return None
+        head, _, last = lin.rpartition(" + ")
+        if last != self.var or re.search(rf"\b{self.var}\b", head):
+            return None
+        self.vectors.append(name)
+        return f"{head} + {self.var}0" if head else f"{self.var}0"
+
+    def vector_context(self, root, coords, tag, var, width):
+        """``context`` for a loop over vectors of ``width``: (lines ahead of the elements, lines
+        per element ``u``, tensors read as vectors)."""
+        self.vec, self.var, self.pre, self.vectors = width, var, [], []
+        try:
+            lines = self.context(root, coords, tag)
+            return self.pre, lines, self.vectors
+        finally:
+            self.vec = 0
 
     def _canon(self, v, coords):
         return tuple("0" if size == 1 else c for size, c in zip(self.shapes[id(v)], coords))
@@ -967,9 +1010,21 @@ class _TileEmitter(_Emitter):
             name, ks = chain
             t = self.tensor_dtype(name)
             st, w, ld, _ = _STORAGE[t]
-            entry = self.plan.level_index(name, ks, _ravel(self.coords[id(v)], self.shapes[id(v)]), self)
+            lin = _ravel(self.coords[id(v)], self.shapes[id(v)])
+            start = self.vector_start(name, ks, lin)
+            if start is not None:  # part of a vector loaded ahead of the unrolled elements
+                vec = f"{self.tag}v{len(self.names)}"
+                self.pre.append(f"      const auto {vec} = nt_ldv<{self.vec}>(p_{name} + ({self.plan.index_expr(name, start)}));")
+                self.define(v, t, f"(({w}){ld.format(f'{vec}.e[u]')})", exact=True)
+                self.masks[id(v)] = frozenset()
+                return
+            entry = self.plan.level_index(name, ks, lin, self)
             ix = f"{self.tag}x{len(self.names)}"
             self.lines.append(f"      const int {ix} = {entry};")
+            if not any(isinstance(k, Value) for k in ks) and self.plan.whole(name):
+                self.define(v, t, f"(({w}){ld.format(f'p_{name}[{ix}]')})", exact=True)
+                self.masks[id(v)] = frozenset()
+                return
             other = self.ctx.views[name].source.other
             other = 0.0 if other is None else float(other)
             o = repr(other) if other == other and abs(other) != float("inf") else (
@@ -1363,6 +1418,8 @@ class TilePlan(GenericPlan):
         self.shapes = _shapes(ctx, values, probe.const_value, self.carried_shapes)
         self.outputs = list(stores)
         self.kernel_name = "nt_generic_tile"
+        self.forms = {}  # tensor -> (element step, whether rows are cut short): see _row_form
+        self.walked = values
         arranged = self.outputs + sorted(
             {_view_chain(e[1])[0] for e in program.effects if e[0] == "view_store"}
             | {_view_chain(v.args[0])[0] for v in values if v.op == "load"
@@ -1399,7 +1456,12 @@ class TilePlan(GenericPlan):
                            for n in self.index_names}
         self.offset_lengths = {(n, d): (_tile_shape(ctx, n)[d] if _tile_shape(ctx, n) else 1) for n, d in self.offsets}
         self.scalar_types = {n: probe.scalar_type(n) for n in self.scalars}
+        self.params = self._params()
+
+    def _params(self):
+        ctx = self.ctx
         params = [f"const int* __restrict__ t_{n}" for n in self.index_names]
+        params += [f"const int* __restrict__ l_{n}" for n in self.index_names if self.forms.get(n, (0, False))[1]]
         params += [f"const int* __restrict__ f_{n}_{d}" for n, d in self.offsets]
         params += [f"const {_STORAGE[_torch_dtype_name(ctx.dtypes[n])][0]}* __restrict__ p_{n}" for n in self.loaded]
         params += [f"{_STORAGE[_torch_dtype_name(ctx.dtypes[n])][0]}* __restrict__ p_{n}"
@@ -1408,7 +1470,7 @@ class TilePlan(GenericPlan):
                    for n in self.raw]
         params += [f"{_STORAGE[self.scalar_types[n]][0]} s_{n}" for n in self.scalars]
         params.append("long long programs")
-        self.params = params
+        return params
 
     def _settle_shapes(self, values, probe):
         """Shape of every loop-carried value: its initial value's, broadcast with its updated
@@ -1523,42 +1585,108 @@ class TilePlan(GenericPlan):
         if w == "bool":
             raise LoweringError("reductions of booleans are not supported")
         ident, comb = self._combine(kind, t, w)
-        val = em.operand(operand, t)
-        mask = em.mask_of(operand)
-        term = f"({mask}) ? {val} : {ident}" if mask else val
-        lanes = 1 if n_out >= 256 else min(64, 1 << int(np.log2(256 // n_out)))
+
+        def accumulate():
+            val = em.operand(operand, t)
+            mask = em.mask_of(operand)
+            term = f"({mask}) ? {val} : {ident}" if mask else val
+            return f"acc = {comb.format(a='acc', b=f'({term})')};"
+
+        step_scalar = accumulate()
+        # A single long reduction takes the whole workgroup (each wave's result through LDS).
+        block = n_out == 1 and extent >= 256
+        lanes = 256 if block else (1 if n_out >= 256 else min(64, 1 << int(np.log2(256 // n_out))))
         lanes = max(1, min(lanes, 1 << int(np.ceil(np.log2(max(extent, 1))))))
         step = 256 // lanes
         o_pad = -(-n_out // step) * step
         arr = f"red{k}"
+        size = 8 if w in ("double", "long long") else 4
         self.decls.append(f"  __shared__ {w} {arr}[{max(n_out, 1)}];")
-        self.lds_bytes += max(n_out, 1) * (8 if w in ("double", "long long") else 4)
+        self.lds_bytes += max(n_out, 1) * size
+        lane = "tid" if block else "g"
+        first, loops = "0", []
+        width = self._vector_width(em)
+        if width and extent >= width:
+            pre, each, vectors = em.vector_context(operand, coords, f"w{k}_", "l", width)
+            if vectors:
+                bound, first = self._vector_bound(vectors, extent, width, f"n{k}")
+                loops += [
+                    f"          {bound}",
+                    f"          for (int l0 = {lane} * {width}; l0 < {first}; l0 += {lanes * width}) {{",
+                    *["    " + x for x in pre],
+                    "#pragma unroll",
+                    f"          for (int u = 0; u < {width}; ++u) {{",
+                    "            const int l = l0 + u;",
+                    *["    " + x for x in each],
+                    f"            {accumulate()}",
+                    "          }",
+                    "          }",
+                ]
+        if first != str(extent):
+            loops += [
+                f"          for (long long l = {first} + {lane}; l < {extent}LL; l += {lanes}) {{",
+                *["    " + x for x in body],
+                f"            {step_scalar}",
+                "          }",
+            ]
         self.lds[id(r)] = (arr, oshape)
         self.types[id(r)] = t
+        shuffles = [f"        for (int s = {min(lanes, 64) // 2}; s > 0; s >>= 1) "
+                    f"acc = {comb.format(a='acc', b='__shfl_xor(acc, s, 64)')};"] if lanes > 1 else []
+        head = f"    {{  // {kind} over {'all axes' if axis is None else f'axis {axis}'}: {n_out} x {extent}"
+        if block:
+            self.decls.append(f"  __shared__ {w} {arr}_w[4];")
+            total = f"{arr}_w[0]"
+            for i in range(1, 4):
+                total = comb.format(a=total, b=f"{arr}_w[{i}]")
+            return "\n".join([
+                head,
+                "        const long long o = 0;",
+                f"        {w} acc = {ident};",
+                *loops, *shuffles,
+                f"        if ((tid & 63) == 0) {arr}_w[tid >> 6] = acc;",
+                "        __syncthreads();",
+                f"        if (tid == 0) {arr}[o] = {em.round_to(t, total)};",
+                "    }",
+                "    __syncthreads();",
+            ])
         return "\n".join([
-            f"    {{  // {kind} over {'all axes' if axis is None else f'axis {axis}'}: {n_out} x {extent}",
+            head,
             f"      const int g = tid % {lanes};",
             f"      for (int o = tid / {lanes}; o < {o_pad}; o += {step}) {{",
             f"        {w} acc = {ident};",
             f"        if (o < {n_out}) {{",
-            f"          for (long long l = g; l < {extent}LL; l += {lanes}) {{",
-            *["    " + x for x in body],
-            f"            acc = {comb.format(a='acc', b=f'({term})')};",
-            "          }",
+            *loops,
             "        }",
-            *([f"        for (int s = {lanes // 2}; s > 0; s >>= 1) "
-               f"acc = {comb.format(a='acc', b='__shfl_xor(acc, s, 64)')};"] if lanes > 1 else []),
+            *shuffles,
             f"        if (g == 0 && o < {n_out}) {arr}[o] = {em.round_to(t, 'acc')};",
             "      }",
             "    }",
             "    __syncthreads();",
         ])
 
+    def _vector_width(self, em):
+        """Elements per vector of a loop over consecutive elements: 16 bytes of the narrowest
+        tensor addressed without a table, at most 8; 0 when there is none."""
+        sizes = [_SIZES[_torch_dtype_name(self.ctx.dtypes[n])] for n, (step, _) in self.forms.items() if step == 1]
+        return min(8, 16 // min(sizes)) if sizes and min(sizes) <= 8 else 0
+
+    def _vector_bound(self, vectors, extent, width, name):
+        """(C statement, C expression) of the number of elements the vector loop covers: whole
+        vectors inside every vector tensor's row."""
+        cut = [f"lm_{n}" for n in dict.fromkeys(vectors) if self.forms[n][1]]
+        if not cut:
+            return "", str(extent // width * width)
+        expr = str(extent)
+        for c in cut:
+            expr = f"min({expr}, {c})"
+        return f"const int {name} = {expr} / {width} * {width};", name
+
     def _staged_stores(self, em):
         """Every stored tile computed into LDS (in its storage type), one barrier, then written."""
         compute, write = [], []
         for out, v in self.stores.items():
-            lines = self._store_block(em, out, v).split("\n")
+            lines = self._store_block(em, out, v, vectors=False).split("\n")
             st = _STORAGE[_torch_dtype_name(self.ctx.dtypes[out])][0]
             n_tile = int(np.prod(_tile_shape(self.ctx, out)) or 1)
             arr = f"stage_{out}"
@@ -1637,7 +1765,7 @@ class TilePlan(GenericPlan):
         self.types[id(v)] = "float32"
         return "\n".join(lines)
 
-    def _store_block(self, em, out, v):
+    def _store_block(self, em, out, v, vectors=True):
         ctx = self.ctx
         tshape = _tile_shape(ctx, out)
         sv = self.shapes[id(v)]
@@ -1645,21 +1773,51 @@ class TilePlan(GenericPlan):
             raise LoweringError(f"a value of shape {sv} is stored to a tile of shape {tshape}")
         n_tile = int(np.prod(tshape)) if tshape else 1
         oc = _unravel("j", tshape)
-        body = em.context(v, oc[len(oc) - len(sv):] if sv else (), f"s{out}_")
+        coords = oc[len(oc) - len(sv):] if sv else ()
         t = _torch_dtype_name(ctx.dtypes[out])
-        src = em.type_of(v)
-        src = "float32" if src == "weak" else src
-        val = em.operand(v, src) if em.is_const(v) else em.names[id(v)]
-        if em.work(src) != em.work(t):
-            val = f"(({em.work(t)}){val})"
-        return "\n".join([
-            f"    for (long long j = tid; j < {n_tile}LL; j += 256) {{",
-            f"      const int oi = {self.index_expr(out, 'j')};",
-            "      if (oi < 0) continue;",
-            *body,
-            f"      p_{out}[oi] = {_STORAGE[t][3].format(val)};",
-            "    }",
-        ])
+
+        def stored():
+            src = em.type_of(v)
+            src = "float32" if src == "weak" else src
+            val = em.operand(v, src) if em.is_const(v) else em.names[id(v)]
+            if em.work(src) != em.work(t):
+                val = f"(({em.work(t)}){val})"
+            return _STORAGE[t][3].format(val)
+
+        lines, first = [], "0"
+        width = self._vector_width(em) if vectors and self.forms.get(out, (0, None))[0] == 1 else 0
+        if width and n_tile >= width:
+            pre, each, read = em.vector_context(v, coords, f"z{out}_", "j", width)
+            bound, first = self._vector_bound(read + [out], n_tile, width, f"n_{out}")
+            lines += [
+                f"    {{  // `{out}`, {width} elements per lane",
+                f"    {bound}",
+                f"    for (int j0 = tid * {width}; j0 < {first}; j0 += {256 * width}) {{",
+                *pre,
+                f"      nt_vec<{_STORAGE[t][0]}, {width}> ov;",
+                "#pragma unroll",
+                f"      for (int u = 0; u < {width}; ++u) {{",
+                "      const int j = j0 + u;",
+                *each,
+                f"      ov.e[u] = {stored()};",
+                "      }",
+                f"      nt_stv(p_{out} + ({self.index_expr(out, 'j0')}), ov);",
+                "    }",
+            ]
+        if first != str(n_tile):
+            body = em.context(v, coords, f"s{out}_")
+            start = "tid" if first == "0" else f"{first} + tid"
+            lines += [
+                f"    for (long long j = {start}; j < {n_tile}LL; j += 256) {{",
+                f"      const int oi = {self.index_expr(out, 'j')};",
+                "      if (oi < 0) continue;",
+                *body,
+                f"      p_{out}[oi] = {stored()};",
+                "    }",
+            ]
+        if width and n_tile >= width:
+            lines.append("    }")
+        return "\n".join(lines)
 
     def _carried_write(self, em, i, n, v, tag, buffer):
         """Lines writing value ``v`` to every element of loop ``i``'s carried ``n`` in ``buffer``."""
@@ -1711,8 +1869,16 @@ class TilePlan(GenericPlan):
         lines.append(f"    const long long po{i} = (n{i} > 0 ? n{i} : 0) & 1;")
         return ["\n".join(lines)]
 
+    def whole(self, name):
+        """Whether every element of ``name``'s tiles lies in the tensor, at a known step."""
+        return name in self.forms and not self.forms[name][1]
+
     def index_expr(self, name, lin):
-        return f"t_{name}[pb_{name} + {lin}]"
+        if name not in self.forms:
+            return f"t_{name}[pb_{name} + {lin}]"
+        step, cut = self.forms[name]
+        at = f"bs_{name}" if step == 0 else f"bs_{name} + (int)({lin}) * {step}" if step != 1 else f"bs_{name} + (int)({lin})"
+        return f"(({lin}) < lm_{name} ? {at} : -1)" if cut else at
 
     def level_index(self, name, ks, inner, em):
         """C index-table entry of element ``inner`` of the level of ``name`` reached by the
@@ -1817,7 +1983,33 @@ class TilePlan(GenericPlan):
         ])
 
     def sources_for(self, values):
-        return [self.source()]
+        return [self.launch_spec(values)[0]]
+
+    @staticmethod
+    def _row_form(table, programs):
+        """``table`` ([programs][tile] offsets, -1 masked) as base[p] + j * step for j < limit[p],
+        masked from there on: (step, base, limit or None when no tile is cut), or None where it is
+        not of that form.  Such a tensor needs one base (and limit) per program instead of an
+        entry per element, and its loads can be vectors.  A tile program is bound by its bytes:
+        a bf16 norm of [2048, 4096] read 4 bytes of table per element and tensor, twice, moved 2
+        bytes per lane and summed on one wave of four, 68.0 us (0.5 TB/s); with rows, 16-byte
+        vectors and all four waves summing 9.2 us (3.6 TB/s)."""
+        if programs <= 0 or table.size == 0 or table.size % programs:
+            return None
+        rows = table.reshape(programs, -1)
+        valid = rows >= 0
+        limit = np.count_nonzero(valid, axis=1).astype(np.int32)
+        j = np.arange(rows.shape[1], dtype=np.int32)
+        whole = bool((limit == rows.shape[1]).all())
+        if not whole and not np.array_equal(valid, j[None, :] < limit[:, None]):
+            return None
+        long = int(np.argmax(limit))
+        step = int(rows[long, 1]) - int(rows[long, 0]) if limit[long] > 1 else 0
+        base = np.where(limit > 0, rows[:, 0], 0).astype(np.int32)
+        expected = base[:, None] + (j.astype(np.int64) * step).astype(np.int32)[None, :]
+        if not np.array_equal(rows if whole else np.where(valid, rows, 0), expected if whole else np.where(valid, expected, 0)):
+            return None
+        return step, base, None if whole else limit
 
     @staticmethod
     def _combine(kind, t, w):
@@ -1836,7 +2028,9 @@ class TilePlan(GenericPlan):
         return (f"(-{inf})" if kind == "max" else inf), f + "({a}, {b})"
 
     def source(self, linear=None, linear_offsets=()):
-        bases = [f"    const long long pb_{n} = p * {self.tile_sizes[n]}LL;" for n in self.tile_sizes]
+        bases = [f"    const long long pb_{n} = p * {self.tile_sizes[n]}LL;" for n in self.tile_sizes if n not in self.forms]
+        bases += [f"    const int bs_{n} = t_{n}[p];" for n in self.forms]
+        bases += [f"    const int lm_{n} = l_{n}[p];" for n, (_, cut) in self.forms.items() if cut]
         bases += [f"    const long long pbo_{n}_{d} = p * {self.offset_lengths[(n, d)]}LL;" for n, d in self.offsets]
         return (
             _PRELUDE
@@ -1855,17 +2049,37 @@ class TilePlan(GenericPlan):
     def launch_spec(self, values):
         """As GenericPlan.launch_spec: the tables, the tensors (loaded, stored, read through
         pointers), the scalars and the number of programs."""
-        maps, args = {}, []
+        maps, tables, forms = {}, {}, {}
+        # A call with a jagged tensor rebuilds its tables every time: they stay tables, so that
+        # its source (and code object) does not follow each batch's rows.
+        plain = not any(jagged.is_jagged(values[n]) for n in self.index_names)
         for n in self.index_names:
             maps[n] = self._maps(n)
-            args.append(("table", self._table(n, values[n], maps[n])[0]))
+            tables[n] = self._table(n, values[n], maps[n])[0]
+            form = self._row_form(tables[n], self.programs) if plain else None
+            if form is not None:
+                forms[n] = form
+                tables[n] = form[1]
+        args = [("table", tables[n]) for n in self.index_names]
+        args += [("table", forms[n][2]) for n in self.index_names if n in forms and forms[n][2] is not None]
         args += [("table", self._tile_offsets(n, d, maps.get(n))) for n, d in self.offsets]
         args += [("tensor", n) for n in self.loaded]
         args += [("tensor", n) for n in self.outputs + self.view_targets]
         args += [("tensor", n) for n in self.raw]
         args += [("scalar", n, "int64" if self.scalar_types[n] == "int64" else "float32") for n in self.scalars]
         args.append(("i64", self.programs))
-        return self.source(), min(self.programs, 256 * 64), args
+        shaped = self._shaped({n: (form[0], form[2] is not None) for n, form in forms.items()})
+        return shaped.source(), min(self.programs, 256 * 64), args
+
+    def _shaped(self, forms):
+        """This plan emitted for tensors of these row forms (the plan itself is not touched)."""
+        if not forms:
+            return self
+        plan = copy.copy(self)
+        plan.forms = forms
+        plan._emit(plan.walked)
+        plan.params = plan._params()
+        return plan
 
     def _tile_offsets(self, name, dim, maps=None):
         """``offsets(dim)`` per program: the source index along ``dim`` of the tile's elements

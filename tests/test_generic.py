@@ -1201,3 +1201,65 @@ def test_output_assigned_in_an_unrolled_loop():
     out = torch.empty_like(x)
     kernel(x, out, BS=128)
     torch.testing.assert_close(out, x * 2.0 + 2)
+
+
+# ------------------------------------------------------------------ rows addressed without tables
+@pytest.mark.parametrize("programs, tile", ((1, 1), (3, 1), (1, 9), (5, 8)))
+def test_row_forms_reproduce_their_tables(programs, tile):
+    # Every table a form is found for is exactly base + j * step below the limit and masked past
+    # it; tables of any other shape keep their entries.
+    from ninetoothed_amd.generic import TilePlan
+
+    rng = np.random.default_rng(programs * 100 + tile)
+    j = np.arange(tile)
+    for step in (0, 1, 3, -2):
+        for cut in (False, True):
+            base = rng.integers(50, 1000, programs)
+            limit = rng.integers(0, tile + 1, programs) if cut else np.full(programs, tile)
+            table = np.where(j[None] < limit[:, None], base[:, None] + j[None] * step, -1).astype(np.int32)
+            form = TilePlan._row_form(table.reshape(-1), programs)
+            assert form is not None
+            got_limit = np.full(programs, tile) if form[2] is None else form[2]
+            again = np.where(j[None] < got_limit[:, None], form[1][:, None] + j[None] * form[0], -1)
+            assert np.array_equal(again, table)
+    if tile > 2:
+        bent = np.tile(np.arange(tile, dtype=np.int32), (programs, 1))
+        bent[-1, -1] += 1
+        assert TilePlan._row_form(bent.reshape(-1), programs) is None
+        holed = np.tile(np.arange(tile, dtype=np.int32), (programs, 1))
+        holed[0, 1] = -1
+        assert TilePlan._row_form(holed.reshape(-1), programs) is None
+
+
+def scaled_norm_application(x, w, out):
+    x32 = ntl.cast(x, ntl.float32)
+    mean_square = ntl.sum(x32 * x32, axis=1) / x.shape[1]
+    out = x32 * ntl.rsqrt(mean_square[:, None] + 1e-6) * ntl.cast(w, ntl.float32)  # noqa: F841
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", (torch.bfloat16, torch.float32))
+@pytest.mark.parametrize("rows, cols, width", ((3, 1, 1), (5, 7, 7), (4, 255, 256), (2, 256, 256), (3, 257, 257),
+                                               (2, 4099, 4100), (700, 2048, 2048), (6, 1000, 128)))
+def test_row_programs_at_vector_edges(rows, cols, width, dtype):
+    # Vectors and their remainder: rows shorter than a vector, one past a vector, cut short by
+    # the tensor's edge, several tiles a row; rows at odd offsets, a broadcast weight, an input
+    # of every other column (no vectors) and an output of another type.
+    kernel = ninetoothed.make(lambda x, w, o: tuple(t.tile((1, WIDTH)) for t in (x, w, o)), scaled_norm_application,
+                              tuple(Tensor(2) for _ in range(3)))
+    g = torch.Generator().manual_seed(cols)
+    wide = torch.randn((rows, 2 * cols + 3), generator=g).to(dtype).cuda()
+    weight = torch.randn((cols,), generator=g).to(dtype).cuda().expand(rows, cols)
+    for x in (wide[:, 1:cols + 1], wide[:, 0:2 * cols:2], wide[:, :cols].contiguous()):
+        for out_dtype in (dtype, torch.float16):
+            buf = torch.full((rows, cols + 2), 7.0, dtype=out_dtype, device="cuda")
+            out = buf[:, 1:cols + 1]
+            kernel(x, weight, out, WIDTH=width)
+            ref = torch.empty((rows, cols), dtype=torch.float64)
+            for c in range(0, cols, width):  # a masked element counts as zero, the mean is over the whole tile
+                xc = x[:, c:c + width].double().cpu()
+                ref[:, c:c + width] = xc * torch.rsqrt((xc * xc).sum(1, keepdim=True) / width + 1e-6)
+            ref *= weight.double().cpu()
+            tol = 1e-5 if out_dtype == torch.float32 else (2e-3 if out_dtype == torch.float16 else 1e-2)
+            assert torch.allclose(out.double().cpu(), ref, atol=tol, rtol=tol)
+            assert torch.all(buf[:, 0] == 7.0) and torch.all(buf[:, -1] == 7.0)
