@@ -245,6 +245,16 @@ int nt_gemm_e4m3(const void* a, int64_t sa_m, int64_t sa_k, const void* b, int64
  * the stream: one argument instead of 20). */
 int nt_gemm_packed(const int64_t* v);
 
+/* The same with a workspace, for fp16/bf16 operands (v[0] 0 or 1, v[20] 0; other calls go to
+ * nt_gemm_packed): v[22] the workspace (256-byte aligned), v[23] its bytes.  It holds fp32
+ * partials where few output tiles make the reduction worth splitting, and aligned copies of
+ * operands whose rows are not 16-byte aligned or whose K (or a row-major b's N) is no multiple
+ * of 8; nothing between calls.  nt_gemm_workspace_size gives the bytes the packed call v[0..21]
+ * wants (0: none; the data pointers count, for their alignment); with fewer the call runs as
+ * nt_gemm_packed. */
+int64_t nt_gemm_workspace_size(const int64_t* v);
+int nt_gemm_packed_ws(const int64_t* v);
+
 /* ---------------------------------------------------------------------------
  * 2-D convolution as an implicit GEMM (cross-correlation, as F.conv2d):
  *   y[n,k,p,q] = cast_y(round(sum_{c,r,s} x[n,c,p*sh - ph + r*dh, q*sw - pw + s*dw] * w[k,c,r,s]))

@@ -67,6 +67,8 @@ _SIGNATURES = {
         for t in ("f16", "bf16")
     },
     "nt_gemm_packed": (_I64P,),
+    "nt_gemm_packed_ws": (_I64P,),
+    "nt_gemm_workspace_size": (_I64P,),
     "nt_conv2d_workspace_size": (_I64,) * 9 + (_I,),
     **{
         f"nt_conv2d_noalloc_{t}": (_P, _I64P, _P, _I64P, _P, _I64P, _I) + (_I64,) * 15 + (_I, _P)
@@ -101,7 +103,7 @@ _SIGNATURES = {
     "nt_rtc_launch": (_P, ctypes.c_uint32, ctypes.c_uint32, ctypes.POINTER(_P), _P),
 }
 _RESTYPES = {"nt_conv2d_workspace_size": ctypes.c_int64, "nt_attention_workspace_size": ctypes.c_int64,
-             "nt_rtc_free": None}
+             "nt_gemm_workspace_size": ctypes.c_int64,              "nt_rtc_free": None}
 
 _lock = threading.Lock()
 _library = None

@@ -20,6 +20,7 @@
 //   16 x 16 block with v_mfma_f32_16x16x4f32, K staged through LDS 256 at a time.
 #include "mfma_core.h"
 
+#include <algorithm>
 #include <cstring>
 #include <type_traits>
 
@@ -44,6 +45,14 @@ struct GemmArgs {
   // gemm_dma128_kernel only: product blockIdx.y of a batch, its a, b and out at these element
   // strides from the first's (0 outside a batch).
   int64_t sa_b, sb_b, so_b;
+  // gemm_dma128_kernel<T, BT, PART>: split blockIdx.z takes kt_per 32-deep k-tiles and stores its
+  // sums, fp32, to part[split][M][Np].
+  float* part;
+  int kt_per;
+  int64_t Np;
+  // A row-major b's rows and columns: K and N, or fewer rows where a is padded along k and b is
+  // not (zeros past them), or more columns where b's rows are padded.
+  int64_t Kb, Nb;
 };
 
 // Map a linear workgroup id to an output tile so that consecutive ids on one XCD
@@ -630,12 +639,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // outputs past N (never stored).  With K not a multiple of 32, the chunks of a past K in
   // the last k-tile are fetched from offset a_end (zeros): an a value past K would otherwise
   // be the next row's, and an infinity there times a zero of b is not zero.
-  const int rows_a = (int)(g.M - m0 < GB_M ? g.M - m0 : GB_M), cols_b = (int)(g.N - n0 < GB_N ? g.N - n0 : GB_N);
+  const int rows_a = (int)(g.M - m0 < GB_M ? g.M - m0 : GB_M), cols_b = (int)min((BT ? g.N : g.Nb) - n0, (int64_t)GB_N);
   const uint32_t a_end = (uint32_t)(((rows_a - 1) * g.sa_m + g.K) * 2);
   const u32x4 rsA = dma::rsrc((const uint16_t*)g.a + m0 * g.sa_m, a_end);
   // b^T (BT) ends at its last valid row (column of b) like a; its chunks past K in the last
   // k-tile read zeros the same way.
-  const uint32_t b_end = BT ? (uint32_t)(((cols_b - 1) * g.sb_n + g.K) * 2) : (uint32_t)(((g.K - 1) * g.sb_k + cols_b) * 2);
+  const uint32_t b_end = BT ? (uint32_t)(((cols_b - 1) * g.sb_n + g.K) * 2) : (uint32_t)(((g.Kb - 1) * g.sb_k + cols_b) * 2);
   const u32x4 rsB = dma::rsrc((const uint16_t*)g.b + (BT ? n0 * g.sb_n : n0), b_end);
   // Load q (0, 1) of this wave per k-tile: a rows 32 wave + 16 q + lane / 4, LDS chunk
   // lane % 4; b rows 4 wave + 2 q + lane / 32, LDS bytes (lane % 32) * 16 of the row (BT:
@@ -789,7 +798,9 @@ constexpr int STAGE = 8192, B0 = 32768, EPI = 65536, LDS = EPI + 4 * 4096;
 __device__ __forceinline__ int bsw(int k) { return k & 3; }
 }  // namespace dma128
 
-template <typename T, bool BT = false>
+// PART: the reduction split over blockIdx.z (few tiles: 64 of them would leave three CUs of four
+// idle), each split's sums to the workspace; gemm_part_kernel adds them and finishes any out.
+template <typename T, bool BT = false, bool PART = false>
 __global__ __launch_bounds__(256) void gemm_dma128_kernel(GemmArgs g) {
   __shared__ __attribute__((aligned(1024))) char lds[dma128::LDS];
   if (blockIdx.y) {  // product blockIdx.y of a batch (no c)
@@ -807,14 +818,15 @@ __global__ __launch_bounds__(256) void gemm_dma128_kernel(GemmArgs g) {
   tile_of(blockIdx.x, g.tiles_m, g.tiles_n, tm, tn);
   const int64_t m0 = (int64_t)tm * TM, n0 = (int64_t)tn * TN;
   const int nk = (int)((g.K + 31) / 32);
+  const int kt0 = PART ? (int)blockIdx.z * g.kt_per : 0, kt1 = PART ? min(nk, kt0 + g.kt_per) : nk;
 
   // Buffer resources end at each panel's last valid element, as in gemm_dma_kernel: rows of a
   // past M and rows of b past K read zeros; the chunks of a (and b^T) past K in the last
   // k-tile are fetched from the resource's end.
-  const int rows_a = (int)(g.M - m0 < TM ? g.M - m0 : TM), cols_b = (int)(g.N - n0 < TN ? g.N - n0 : TN);
+  const int rows_a = (int)(g.M - m0 < TM ? g.M - m0 : TM), cols_b = (int)min((BT ? g.N : g.Nb) - n0, (int64_t)TN);
   const uint32_t a_end = (uint32_t)(((rows_a - 1) * g.sa_m + g.K) * 2);
   const u32x4 rsA = dma::rsrc((const uint16_t*)g.a + m0 * g.sa_m, a_end);
-  const uint32_t b_end = BT ? (uint32_t)(((cols_b - 1) * g.sb_n + g.K) * 2) : (uint32_t)(((g.K - 1) * g.sb_k + cols_b) * 2);
+  const uint32_t b_end = BT ? (uint32_t)(((cols_b - 1) * g.sb_n + g.K) * 2) : (uint32_t)(((g.Kb - 1) * g.sb_k + cols_b) * 2);
   const u32x4 rsB = dma::rsrc((const uint16_t*)g.b + (BT ? n0 * g.sb_n : n0), b_end);
   int va[2], vb[2], va_last[2], vb_last[2];
 #pragma unroll
@@ -889,13 +901,13 @@ __global__ __launch_bounds__(256) void gemm_dma128_kernel(GemmArgs g) {
   floatx16 acc[2][2];
   zero_acc(acc);
 
-  // nk >= 3 (the launcher checks): tiles 0..2 in flight, wait for tile 0.
-  for (int kt = 0; kt < 3; ++kt)
+  // kt1 - kt0 >= 3 (the launcher checks): three tiles in flight, wait for the first.
+  for (int kt = kt0; kt < kt0 + 3; ++kt)
     for (int u = 0; u < 4; ++u) load_unit(u, kt);
   asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
   __builtin_amdgcn_s_barrier();
 #pragma unroll
-  for (int x = 0; x < 4; ++x) read_unit(x, 0, 0);
+  for (int x = 0; x < 4; ++x) read_unit(x, 0, (kt0 % dma::STAGES) * dma128::STAGE);
 
 #define NT_FENCE() __builtin_amdgcn_sched_barrier(0)
   // One k-tile, as gemm_dma_kernel's: HAS1 reads the next tile's slice 0 during slice 1, LOAD
@@ -931,13 +943,103 @@ __global__ __launch_bounds__(256) void gemm_dma128_kernel(GemmArgs g) {
   using V4 = std::integral_constant<int, 4>;
   using V0 = std::integral_constant<int, 0>;
   using VN = std::integral_constant<int, -1>;
-  int kt = 0;
-  for (; kt + 3 < nk; ++kt) step(T1{}, T1{}, V4{}, kt);
+  int kt = kt0;
+  for (; kt + 3 < kt1; ++kt) step(T1{}, T1{}, V4{}, kt);
   step(T1{}, F1{}, V4{}, kt);
   step(T1{}, F1{}, V0{}, kt + 1);
   step(F1{}, F1{}, VN{}, kt + 2);
 
+  if constexpr (PART) {
+    // a register of the wave holds two rows of 32 consecutive columns: 128-byte runs
+    float* P = g.part + (int64_t)blockIdx.z * g.M * g.Np;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int64_t col = n0 + wn * 64 + j * 32 + (lane & 31);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int64_t row = m0 + wm * 64 + i * 32 + acc_row(r, lane);
+          if (row < g.M && col < g.Np) P[row * g.Np + col] = acc[i][j][r];
+        }
+      }
+    return;
+  }
   dma_fast_epilogue<2, true, 2, dma128::EPI>(g, acc, lds, wave, lane, m0 + wm * 64, n0 + wn * 64);
+}
+
+// Sums the splits of gemm_dma128_kernel<.., PART> and finishes: out = beta c + alpha round(sum),
+// any strides and types; a lane takes four consecutive columns of a row, four splits' loads in
+// flight, summed in the order of the splits.
+__global__ __launch_bounds__(256) void gemm_part_kernel(GemmArgs g, int splits) {
+  const int64_t nv = g.Np / 4, total = g.M * nv, step = g.M * g.Np;
+  const bool vec = g.out_dtype != NT_DTYPE_F32 && g.so_n == 1 && g.so_m % 4 == 0 && (uintptr_t)g.out % 8 == 0;
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < total; e += (int64_t)gridDim.x * 256) {
+    const int64_t row = e / nv, col = (e - row * nv) * 4;
+    const float* src = g.part + row * g.Np + col;
+    floatx4 v = {0.f, 0.f, 0.f, 0.f};
+    int sp = 0;
+    for (; sp + 4 <= splits; sp += 4) {
+      floatx4 a[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) a[i] = *(const floatx4*)(src + (sp + i) * step);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v += a[i];
+    }
+    for (; sp < splits; ++sp) v += *(const floatx4*)(src + sp * step);
+    float r[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      r[u] = g.alpha * round_through(v[u], g.round_dtype);
+      if (g.c && col + u < g.N) r[u] += g.beta * load_c<false>(g, row * g.sc_m + (col + u) * g.sc_n);
+    }
+    if (vec && col + 4 <= g.N) {
+      uint16_t o[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) o[u] = g.out_dtype == NT_DTYPE_F16 ? float_to_f16_bits(r[u]) : float_to_bf16_bits(r[u]);
+      *(u32x2*)((uint16_t*)g.out + row * g.so_m + col) = *(const u32x2*)o;
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (col + u < g.N) store_from_float(g.out, row * g.so_m + (col + u) * g.so_n, g.out_dtype, r[u]);
+    }
+  }
+}
+
+// Rows of 16-bit elements at any alignment and row stride copied to rows of Lp (a multiple of 8)
+// elements, zeros past L and in rows past `rows`, so that the DMA kernels can take operands they
+// could not (an odd K or N, a view off a 16-byte boundary): 16 bytes per lane, read unaligned.
+// Two operands in one launch: the first b0 workgroups' worth of chunks are the first's.
+namespace skinny {
+constexpr int KC = 64;  // k per chunk: one 128-byte line of a row
+struct __attribute__((packed, aligned(2))) unaligned16 {
+  u32x4 v;
+};
+}  // namespace skinny
+struct PadRows {
+  const uint16_t* src;
+  uint16_t* dst;
+  int64_t rows, stride, L, Lp, chunks;  // chunks: 16-byte pieces of dst (0: nothing to copy)
+};
+__global__ __launch_bounds__(256) void gemm_pad_kernel(PadRows p0, PadRows p1) {
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < p0.chunks + p1.chunks; e += (int64_t)gridDim.x * 256) {
+    const bool second = e >= p0.chunks;
+    const PadRows& p = second ? p1 : p0;
+    const int64_t c = second ? e - p0.chunks : e, per = p.Lp / 8;
+    const int64_t row = c / per, k = (c - row * per) * 8;
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (row < p.rows && k < p.L) {
+      const uint16_t* s = p.src + row * p.stride + k;
+      if (k + 8 <= p.L) {
+        v = ((const skinny::unaligned16*)s)->v;
+      } else {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (k + u < p.L) v[u >> 1] |= (uint32_t)s[u] << (16 * (u & 1));
+      }
+    }
+    *(u32x4*)(p.dst + c * 8) = v;
+  }
 }
 
 // Few rows (M <= 64) against k-contiguous b (b^T rows, x @ w.t(): a linear layer on a few
@@ -952,10 +1054,6 @@ __global__ __launch_bounds__(256) void gemm_dma128_kernel(GemmArgs g) {
 // may be anything: only the last, partial chunk of K is loaded element by element.  Rows
 // past M and columns past N read row 0 and are never stored.
 namespace skinny {
-constexpr int KC = 64;  // k per chunk: one 128-byte line of a row
-struct __attribute__((packed, aligned(2))) unaligned16 {
-  u32x4 v;
-};
 template <typename T>
 struct mma16;
 template <>
@@ -1465,8 +1563,148 @@ __global__ void gemm_k0_kernel(GemmArgs g) {
 // 128-wide kernel wins up to 128 such tiles (2048^3 729 against 412 TFLOP/s, 8192 x 1024 x
 // 8192 814 against 770) and loses from 144 (3072^3 681 against 849).
 constexpr int64_t DMA128_BELOW = 136;
+
+// The route of a 16-bit product through a workspace (config 0):
+//   - a reduction split over workgroups, for outputs of few 128 x 128 tiles;
+//   - operands that the DMA kernels cannot read where they are (rows off a 16-byte boundary, K
+//     or a row-major b's N no multiple of 8, K below 96) copied into aligned, zero-padded rows;
+//   - an out that the 128-wide kernel's epilogue cannot store, through the fp32 partials.
+// bf16 us with weights rotated past the caches, split / before / torch: 200 x 4096 x 4096 22.8 /
+// 51.3 / 22.2, 128 x 4096 x 4096 19.2 / 52.9 / 24.0, 200 x 4096 x 11008 45.2 / 130 / 48.9,
+// 512 x 4096 x 4096 36.5 / 52.5 / 29.7, 1000 x 1024 x 4096 20.8 / 36.1 / 18.7.
+struct Gemm16Route {
+  bool bt, pad_a, pad_b, big, part;
+  int64_t Kp, Nbp, splits, per;          // K as multiplied; a padded b's row length
+  int64_t a_bytes, b_bytes, part_bytes;  // the workspace: padded a, padded b, partials
+  int64_t bytes() const { return a_bytes + b_bytes + part_bytes; }
+};
+// Splits of nk 32-deep k-tiles over `tiles` workgroups, two of which fit a CU: as many as fill
+// the 256 CUs once, or twice where that leaves fewer of them idle (86 tiles: 5 splits 31.9 us, 4
+// 34.0, 2 36.9 at 64 x 11008 x 4096; 64 tiles: 4 splits 22.8, 8 25.4 at 200 x 4096 x 4096), each
+// with at least 8 k-tiles (and the last, what is left, at least 3).
+static int64_t gemm_splits(int64_t tiles, int64_t nk, int64_t* per) {
+  *per = nk;
+  if (tiles > 128 || nk < 64) return 1;
+  const int64_t once = 256 / tiles, twice = 512 / tiles;
+  int64_t sp = twice * tiles * 256 * 100 > once * tiles * 512 * 115 ? twice : once;
+  sp = std::min(sp, nk / 8);
+  for (; sp > 1; --sp) {
+    const int64_t p = cdiv(nk, sp), used = cdiv(nk, p);
+    if (nk - (used - 1) * p >= 3) {
+      *per = p;
+      return used;
+    }
+  }
+  return 1;
+}
+static bool gemm16_out_fast(const GemmArgs& g) {
+  return g.out_dtype != NT_DTYPE_F32 && g.so_n == 1 && g.so_m >= 0 && g.so_m % 8 == 0 && (uintptr_t)g.out % 16 == 0 &&
+         g.N % 8 == 0 &&
+         (!g.c || (g.c_dtype == g.out_dtype && g.sc_n == 1 && g.sc_m >= 0 && g.sc_m % 8 == 0 &&
+                   (uintptr_t)g.c % 16 == 0 && 127 * g.sc_m + 128 <= 0x3fffffffLL));
+}
+// False: no workspace is wanted (or none would help) for this product.
+static bool gemm16_route(const GemmArgs& g, Gemm16Route& r) {
+  if (gemm_check(g) || !valid_dtype(g.c_dtype) || g.M <= 0 || g.N <= 0 || g.K <= 0 || !g.a || !g.b || !g.out) return false;
+  if (g.sa_k != 1 || (g.sb_n != 1 && g.sb_k != 1)) return false;
+  r = Gemm16Route{};
+  r.bt = g.sb_n != 1;
+  const int64_t sb = r.bt ? g.sb_n : g.sb_k;
+  const bool k_odd = g.K % 8 != 0 || g.K < 96;
+  r.Kp = k_odd ? std::max<int64_t>(96, cdiv(g.K, 8) * 8) : g.K;
+  r.Nbp = cdiv(g.N, 8) * 8;
+  r.pad_a = k_odd || g.sa_m < 0 || g.sa_m % 8 != 0 || (uintptr_t)g.a % 16 != 0;
+  r.pad_b = (r.bt ? k_odd : g.N % 8 != 0) || sb < 0 || sb % 8 != 0 || (uintptr_t)g.b % 16 != 0;
+  const int64_t t256 = cdiv(g.M, GB_M) * cdiv(g.N, GB_N), t128 = cdiv(g.M, 128) * cdiv(g.N, 128);
+  if (t128 > 0x7fffffffLL) return false;
+  const bool padded = r.pad_a || r.pad_b, fast = gemm16_out_fast(g);
+  r.big = t256 >= DMA128_BELOW;
+  r.splits = 1;
+  r.per = cdiv(r.Kp, 32);
+  if (!r.big) r.splits = gemm_splits(t128, cdiv(r.Kp, 32), &r.per);
+  // Few rows against b^T rows: the few-rows kernel, which takes any alignment, unless past 32
+  // rows b is long enough for its re-reads of a to cost more than the split's partials (us,
+  // few-rows / split: 64 x 1024 x 1024 9.5 / 9.2, 64 x 4096 x 4096 18.6 / 16.2,
+  // 64 x 11008 x 4096 34.2 / 31.9, 64 x 4096 x 11008 47.0 / 29.1; 20 x 4096 x 4096 12.3 / 14.5).
+  if (g.M <= 64 && g.sb_k == 1 && (padded || r.splits == 1 || g.M <= 32 || g.N * g.K < (1LL << 24)))
+    return false;
+  r.part = !r.big && (r.splits > 1 || !fast);
+  if (!padded && !r.part) return false;  // nothing to gain
+  const int64_t sa = r.pad_a ? r.Kp : g.sa_m, sbp = r.pad_b ? (r.bt ? r.Kp : r.Nbp) : sb;
+  if (255 * sa + r.Kp > 0x3fffffffLL || (r.bt ? 255 * sbp + r.Kp : (r.Kp - 1) * sbp + 256) > 0x3fffffffLL) return false;
+  auto up = [](int64_t b) { return cdiv(b, 256) * 256; };
+  if (r.pad_a) r.a_bytes = up(g.M * r.Kp * 2);
+  if (r.pad_b) r.b_bytes = up((r.bt ? g.N * r.Kp : g.K * r.Nbp) * 2);
+  if (r.part) r.part_bytes = up(r.splits * g.M * r.Nbp * 4);
+  return r.bytes() <= (1LL << 30);
+}
 template <typename T>
-static int gemm16_launch(GemmArgs g, hipStream_t stream, int config = 0) {
+static int gemm16_route_launch(GemmArgs g, const Gemm16Route& r, char* ws, hipStream_t stream) {
+  PadRows pa{}, pb{};
+  if (r.pad_a) pa = PadRows{(const uint16_t*)g.a, (uint16_t*)ws, g.M, g.sa_m, g.K, r.Kp, g.M * (r.Kp / 8)};
+  if (r.pad_b)
+    pb = r.bt ? PadRows{(const uint16_t*)g.b, (uint16_t*)(ws + r.a_bytes), g.N, g.sb_n, g.K, r.Kp, g.N * (r.Kp / 8)}
+              : PadRows{(const uint16_t*)g.b, (uint16_t*)(ws + r.a_bytes), g.K, g.sb_k, g.N, r.Nbp, g.K * (r.Nbp / 8)};
+  if (r.pad_a || r.pad_b) {
+    const int64_t blocks = cdiv(pa.chunks + pb.chunks, 256);
+    hipLaunchKernelGGL(gemm_pad_kernel, dim3((unsigned)(blocks < 16384 ? blocks : 16384)), dim3(256), 0, stream, pa, pb);
+  }
+  g.Kb = g.K;
+  if (r.pad_a) {
+    g.a = ws;
+    g.sa_m = r.Kp;
+  }
+  if (r.pad_b) {
+    g.b = ws + r.a_bytes;
+    if (r.bt)
+      g.sb_n = r.Kp;
+    else
+      g.sb_k = r.Nbp;
+  }
+  if (r.pad_b && !r.bt) g.Nb = r.Nbp;
+  g.K = r.Kp;
+  const bool fast = gemm16_out_fast(g);
+  if (r.big) {
+    g.tiles_m = (int)cdiv(g.M, GB_M);
+    g.tiles_n = (int)cdiv(g.N, GB_N);
+    g.c_pre = fast;
+    const dim3 grid((unsigned)(g.tiles_m * g.tiles_n));
+    if (r.bt && fast)
+      hipLaunchKernelGGL((gemm_dma_kernel<T, true, true>), grid, dim3(512), 0, stream, g);
+    else if (r.bt)
+      hipLaunchKernelGGL((gemm_dma_kernel<T, false, true>), grid, dim3(512), 0, stream, g);
+    else if (fast)
+      hipLaunchKernelGGL((gemm_dma_kernel<T, true>), grid, dim3(512), 0, stream, g);
+    else
+      hipLaunchKernelGGL((gemm_dma_kernel<T, false>), grid, dim3(512), 0, stream, g);
+    return launch_status();
+  }
+  g.tiles_m = (int)cdiv(g.M, 128);
+  g.tiles_n = (int)cdiv(g.N, 128);
+  const dim3 grid((unsigned)(g.tiles_m * g.tiles_n), 1, (unsigned)r.splits);
+  if (!r.part) {
+    g.c_pre = 1;
+    if (r.bt)
+      hipLaunchKernelGGL((gemm_dma128_kernel<T, true>), grid, dim3(256), 0, stream, g);
+    else
+      hipLaunchKernelGGL((gemm_dma128_kernel<T, false>), grid, dim3(256), 0, stream, g);
+    return launch_status();
+  }
+  g.part = (float*)(ws + r.a_bytes + r.b_bytes);
+  g.kt_per = (int)r.per;
+  g.Np = r.Nbp;
+  if (r.bt)
+    hipLaunchKernelGGL((gemm_dma128_kernel<T, true, true>), grid, dim3(256), 0, stream, g);
+  else
+    hipLaunchKernelGGL((gemm_dma128_kernel<T, false, true>), grid, dim3(256), 0, stream, g);
+  const int64_t blocks = cdiv(g.M * (g.Np / 4), 256);
+  hipLaunchKernelGGL(gemm_part_kernel, dim3((unsigned)(blocks < 8192 ? blocks : 8192)), dim3(256), 0, stream, g,
+                     (int)r.splits);
+  return launch_status();
+}
+
+template <typename T>
+static int gemm16_launch(GemmArgs g, hipStream_t stream, int config = 0, void* ws = nullptr, int64_t ws_bytes = 0) {
   if (config < 0 || config > 5) return NT_ERR_INVALID;
   if (int e = gemm_check(g)) return e;
   if (!valid_dtype(g.c_dtype)) return NT_ERR_INVALID;  // an fp8 c goes with fp8 operands
@@ -1478,6 +1716,9 @@ static int gemm16_launch(GemmArgs g, hipStream_t stream, int config = 0) {
   }
   const int64_t tiles_m = cdiv(g.M, GB_M), tiles_n = cdiv(g.N, GB_N);
   if (tiles_m * tiles_n > 0x7fffffffLL) return NT_ERR_INVALID;
+  Gemm16Route route;
+  if (config == 0 && ws && (uintptr_t)ws % 256 == 0 && gemm16_route(g, route) && ws_bytes >= route.bytes())
+    return gemm16_route_launch<T>(g, route, (char*)ws, stream);
   g.tiles_m = (int)tiles_m;
   g.tiles_n = (int)tiles_n;
   // (row strides non-negative: the DMA kernels address panels with unsigned 32-bit offsets)
@@ -1846,7 +2087,7 @@ int gemm16_batch128(int dtype, const void* a, int64_t sa_m, int64_t sa_b, const 
   g.a = a; g.b = b; g.out = out;
   g.sa_m = sa_m; g.sa_k = 1; g.sb_k = sb_k; g.sb_n = 1; g.so_m = so_m; g.so_n = 1;
   g.sa_b = sa_b; g.sb_b = sb_b; g.so_b = so_b;
-  g.M = M; g.N = N; g.K = K;
+  g.M = M; g.N = N; g.K = K; g.Kb = K; g.Nb = N;
   g.alpha = 1.0f; g.beta = 0.0f;
   g.out_dtype = out_dtype; g.c_dtype = out_dtype; g.round_dtype = round_dtype;
   g.tiles_m = (int)cdiv(M, 128);
@@ -1867,7 +2108,7 @@ static GemmArgs make_args(const void* a, int64_t sa_m, int64_t sa_k, const void*
   g.a = a; g.b = b; g.c = c; g.out = out;
   g.sa_m = sa_m; g.sa_k = sa_k; g.sb_k = sb_k; g.sb_n = sb_n;
   g.sc_m = sc_m; g.sc_n = sc_n; g.so_m = so_m; g.so_n = so_n;
-  g.M = M; g.N = N; g.K = K;
+  g.M = M; g.N = N; g.K = K; g.Kb = K; g.Nb = N;
   g.alpha = alpha; g.beta = beta;
   // out_dtype: bits 0-7 out's type; bits 8-15 c's type + 1 (0: c has out's type).
   const int c_field = (out_dtype >> 8) & 0xff;
@@ -1907,6 +2148,35 @@ extern "C" int nt_gemm_e5m2(NT_GEMM_PARAMS) {
 }
 extern "C" int nt_gemm_e4m3(NT_GEMM_PARAMS) {
   return nt::gemm8_launch<nt::src_e4m3>(nt::make_args(NT_GEMM_ARGS), stream);
+}
+
+namespace {
+// The arguments of a GEMM entry point from its packed form.
+nt::GemmArgs unpack_gemm(const int64_t* v) {
+  auto ptr = [&](int i) { return (void*)(intptr_t)v[i]; };
+  auto flt = [&](int i) {
+    const uint32_t bits = (uint32_t)(uint64_t)v[i];
+    float x;
+    std::memcpy(&x, &bits, sizeof(x));
+    return x;
+  };
+  return nt::make_args(ptr(1), v[2], v[3], ptr(4), v[5], v[6], ptr(7), v[8], v[9], ptr(10), v[11], v[12], (int)v[13],
+                       v[14], v[15], v[16], flt(17), flt(18), (int)v[19]);
+}
+}  // namespace
+
+extern "C" int64_t nt_gemm_workspace_size(const int64_t* v) {
+  if (v == nullptr || v[0] < 0 || v[0] > 1 || v[20] != 0) return 0;
+  nt::Gemm16Route r;
+  return nt::gemm16_route(unpack_gemm(v), r) ? r.bytes() : 0;
+}
+extern "C" int nt_gemm_packed_ws(const int64_t* v) {
+  if (v == nullptr) return NT_ERR_INVALID;
+  if (v[0] < 0 || v[0] > 1 || v[20] != 0) return nt_gemm_packed(v);
+  const hipStream_t stream = (hipStream_t)(intptr_t)v[21];
+  void* ws = (void*)(intptr_t)v[22];
+  return v[0] == 0 ? nt::gemm16_launch<nt::f16_t>(unpack_gemm(v), stream, 0, ws, v[23])
+                   : nt::gemm16_launch<nt::bf16_t>(unpack_gemm(v), stream, 0, ws, v[23]);
 }
 
 // The GEMM entry points with their arguments in one int64 array (see nt_mi355x.h).

@@ -334,6 +334,27 @@ def bind_gemm(a, b, out, c=None, round_dtype=None, config=0):
         template = struct.pack("<22q", which, 0, sa_m, sa_k, 0, sb_k, sb_n, 0, sc_m, sc_n, 0, so_m, so_n, out_code, m,
                                n, k, 0, 0, rd, int(config), 0)
         call = _fastkey.call
+        nbytes = 0
+        if which < 2 and not config:
+            sample = list(struct.unpack("<22q", template))
+            for slot, t in zip(_GEMM_POINTER_SLOTS, (a, b, c, out)):
+                sample[slot] = t.data_ptr() if t is not None else 0
+            nbytes = int(_lib.load().nt_gemm_workspace_size((ctypes.c_int64 * 22)(*sample)))
+        if nbytes:
+            import torch
+
+            addr_ws = _packed_address("nt_gemm_packed_ws")
+            template_ws = template + struct.pack("<2q", 0, nbytes)
+
+            def launch(a, b, out, c, alpha, beta):
+                # from torch's stream-ordered caching allocator on every call, as conv2d's
+                ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+                code = call(addr_ws, template_ws, _GEMM_WS_POINTER_SLOTS, (a, b, c, out, ws), _GEMM_VALUE_SLOTS,
+                            (_float_bits(alpha), _float_bits(beta), stream() or 0))
+                if code:
+                    _raise(code, name)
+
+            return launch
 
         def launch(a, b, out, c, alpha, beta):
             code = call(addr, template, _GEMM_POINTER_SLOTS, (a, b, c, out), _GEMM_VALUE_SLOTS,
@@ -356,6 +377,7 @@ def bind_gemm(a, b, out, c=None, round_dtype=None, config=0):
 _PACKED_GEMM_ENTRY = {"nt_gemm_f16": 0, "nt_gemm_bf16": 1, "nt_gemm_f32": 2, "nt_gemm_e5m2": 3, "nt_gemm_e4m3": 4,
                       "nt_gemm_config_f16": 0, "nt_gemm_config_bf16": 1}
 _GEMM_POINTER_SLOTS = (1, 4, 7, 10)
+_GEMM_WS_POINTER_SLOTS = (1, 4, 7, 10, 22)  # nt_gemm_packed_ws: and the workspace (its bytes in slot 23)
 _GEMM_VALUE_SLOTS = (17, 18, 21)
 
 

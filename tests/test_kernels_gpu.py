@@ -462,6 +462,42 @@ def test_gemm_few_rows_unaligned(mnk, dtype):
     assert torch.allclose(out.double(), ref, atol=tol, rtol=tol)
 
 
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("bt", (False, True))
+@pytest.mark.parametrize("mnk", (
+    (65, 128, 2048), (128, 130, 4096), (200, 264, 2080), (100, 72, 5000),  # split reductions, ragged last split
+    (65, 33, 17), (129, 257, 95), (300, 127, 1001), (130, 1, 7), (1, 70, 33), (64, 200, 2049),  # padded operands
+    (3001, 4099, 131), (4096, 2816, 97)))  # ... on 256 x 256 tiles
+def test_gemm_through_a_workspace(mnk, bt, dtype):
+    # The workspace route (split reduction, padded copies of unaligned operands, an out the
+    # 128-wide epilogue cannot store) against fp64 and against the same call with none.  Rows
+    # start off 16-byte boundaries and are followed by infinities, which no product may see.
+    m, n, k = mnk
+    inf = float("inf")
+    abuf = torch.full((m, k + 3), inf, dtype=dtype, device=DEV)
+    a = abuf[:, 1:k + 1] if k % 8 else abuf[:, :k].contiguous()
+    a.copy_(_randn((m, k), dtype, 140, 1.0 / math.sqrt(k)))
+    rows, cols = (n, k) if bt else (k, n)
+    bbuf = torch.full((rows, cols + 5), inf, dtype=dtype, device=DEV)
+    b = bbuf[:, 2:cols + 2] if cols % 8 else bbuf[:, :cols].contiguous()
+    b.copy_(_randn((rows, cols), dtype, 141))
+    b = b.t() if bt else b
+    ref = a.double() @ b.double().contiguous()
+    tol = 1e-2 if dtype == torch.bfloat16 else 2e-3  # the result's rounding at magnitudes up to about 4
+    for out_dtype in (dtype, torch.float32):
+        for c in (None, _randn((1, n), out_dtype, 142).expand(m, n)):
+            want = 0.5 * ref + (2.0 * c.double() if c is not None else 0.0)
+            obuf = torch.full((m, n + 3), 7.0, dtype=out_dtype, device=DEV)
+            out = obuf[:, 1:n + 1]
+            kernels.gemm(a, b, out, c=c, alpha=0.5, beta=2.0)
+            t = 1e-4 if out_dtype == torch.float32 else tol
+            assert torch.allclose(out.double(), want, atol=t, rtol=t)
+            assert torch.all(obuf[:, 0] == 7.0) and torch.all(obuf[:, n + 1:] == 7.0)
+    out = torch.empty((m, n), dtype=dtype, device=DEV)
+    kernels.gemm(a, b, out)
+    assert torch.allclose(out.double(), ref, atol=tol, rtol=tol)
+
+
 def test_gemm_few_rows_rejects_unfit_calls():
     from ninetoothed_amd.errors import KernelLaunchError
 
