@@ -85,8 +85,10 @@ int nt_softmax_bf16(const void* x, int64_t x_row_stride, int64_t x_col_stride,
  * nt_softmax_* plus `config` (0 = as nt_softmax_* choose; 1, 2, 3 = the register path
  * with workgroups of four, eight, one wave, when the segment fits it; 4 = the two-sweep
  * kernel; 5 = a group of lanes per segment, up to four 16-byte vectors per lane of one
- * wave; 6 = the element-wise kernel for any strides).  A forced configuration that does
- * not fit returns NT_ERR_INVALID before launching.  Replaces the reference's tuning over num_warps 4, 8, 1
+ * wave; 6 = the element-wise kernel for any strides; 7, 8 = the segment held as raw 16-byte
+ * vectors, up to 16 a lane, by 256 or 1024 lanes, x and y in one 16-byte phase).  A forced
+ * configuration that does not fit returns NT_ERR_INVALID before launching.  Replaces the
+ * reference's tuning over num_warps 4, 8, 1
  * (reference src/ninetoothed/backends/triton.py:151-155). */
 int nt_softmax_config_f32(const void* x, int64_t x_row_stride, int64_t x_col_stride,
                           void* y, int64_t y_row_stride, int64_t y_col_stride,

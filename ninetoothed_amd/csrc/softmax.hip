@@ -5,7 +5,8 @@
 // registers between the three phases (max, sum of exp, scale), so nothing is
 // re-read; reductions are wave64 butterflies plus one LDS exchange across the four
 // waves.  exp(x) is computed as exp2(x * log2 e) on the hardware v_exp_f32.
-// Segments longer than the register path holds use a two-sweep kernel: an online
+// Segments longer than that, and rows off a 16-byte boundary, are held as raw vectors by up
+// to 1024 lanes; longer ones yet use a two-sweep kernel: an online
 // (max, sum) sweep, then a scaling sweep; segments of at most a few vectors per lane of
 // one wave use a kernel that gives each segment a group of lanes.
 #include "nt_common.h"
@@ -36,11 +37,16 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   const int w = threadIdx.x / 64;
   if ((threadIdx.x & 63) == 0) red[w] = v;
   __syncthreads();
-  float r = red[0];
+  // pairwise: fp32 [2048, 50257] is 5.2e-8 off 64 bits so, 7.3e-8 with sixteen waves' sums in turn
+  float r[NW];
 #pragma unroll
-  for (int i = 1; i < NW; ++i) r += red[i];
+  for (int i = 0; i < NW; ++i) r[i] = red[i];
+#pragma unroll
+  for (int n = NW / 2; n > 0; n /= 2)
+#pragma unroll
+    for (int i = 0; i < n; ++i) r[i] += r[i + n];
   __syncthreads();
-  return r;
+  return r[0];
 }
 
 // Register path: NT lanes per workgroup, each owning VPT vectors of V elements.
@@ -297,6 +303,93 @@ __global__ __launch_bounds__(NT) void softmax_long_kernel(const typename elem<T>
   }
 }
 
+// Segments too long for the register path above, or rows whose 16-byte phase changes from
+// segment to segment: NT lanes hold the whole segment as R raw 16-byte vectors each (64 VGPRs
+// at R = 16, so 1024 lanes stay within 128), read once by bounded buffer loads that are all
+// in flight together, with a head and a tail of single elements.  fp32 keeps the exponentials
+// in place of the elements; 16-bit elements stay raw, their exponentials computed twice.
+// HBM-bound where there are segments enough; with few, one CU's fetch rate and the latency of
+// the three phases.  Measured against the two-sweep kernel, which fetches the segment twice:
+// fp32 [32, 50257] 13.2 -> 9.3 us, [2048, 50257] 229 -> 161 (5.1 TB/s), fp16 [2048, 50257]
+// 103 -> 77; against the register path's element loads: bf16 [4096, 5001] 59.5 -> 19.8, fp16
+// [4096, 16001] 179 -> 42, fp32 [32, 12345] 7.9 -> 4.7.
+template <typename T, int NT, int R>
+__global__ __launch_bounds__(NT) void softmax_hold_kernel(const typename elem<T>::storage* __restrict__ x, int64_t xs,
+                                                          typename elem<T>::storage* __restrict__ y, int64_t ys,
+                                                          int64_t cols, int64_t block, int64_t segs_per_row) {
+  typedef typename elem<T>::storage S;
+  constexpr int V = 16 / sizeof(S);
+  constexpr uint32_t NEG = elem<T>::code == NT_DTYPE_F32 ? 0xff800000u : elem<T>::code == NT_DTYPE_F16 ? 0xfc00fc00u : 0xff80ff80u;
+  // Widened 16-bit elements are kept from one phase to the next where they fit (bf16
+  // [4096, 5001]: 19.8 us, widened anew 22.8); at 1024 lanes and R = 16 they would spill.
+  constexpr bool ANEW = NT == 1024 && R == 16;
+  __shared__ float red[NT / 64];
+  const int64_t seg = blockIdx.x;
+  const int64_t row = seg / segs_per_row;
+  const int64_t c0 = (seg % segs_per_row) * block;
+  const int len = (int)((cols - c0 < block) ? (cols - c0) : block);
+  const S* xr = x + row * xs + c0;
+  S* yr = y + row * ys + c0;
+  const int head = seg_head<S, true>(xr, len);
+  const int nvec = (len - head) / V, tail = len - head - nvec * V;
+  const S* xb = xr + head;
+  S* yb = yr + head;
+  const int t = threadIdx.x;
+  const float hv = t < head ? elem<T>::to_float(xr[t]) : -INFINITY;
+  const float tv = t < tail ? elem<T>::to_float(xb[nvec * V + t]) : -INFINITY;
+  // bounded by the segment's last whole vector: the loads beyond it read zeros
+  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)xb, 0, nvec * 16, 0x00020000);
+  u32x4 raw[R];
+#pragma unroll
+  for (int j = 0; j < R; ++j) raw[j] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (j * NT + t) * 16, 0, 0);
+  float mx = fmaxf(hv, tv);
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    if (j * NT + t >= nvec) raw[j] = u32x4{NEG, NEG, NEG, NEG};
+    const S* p = (const S*)&raw[j];
+#pragma unroll
+    for (int u = 0; u < V; ++u) mx = fmaxf(mx, elem<T>::to_float(p[u]));
+  }
+  mx = block_max<NT / 64>(mx, red);
+  const float he = fast_exp(hv - mx), te = fast_exp(tv - mx);
+  float part[2] = {t < head ? he : 0.f, t < tail ? te : 0.f};
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    if constexpr (ANEW) asm volatile("" : "+v"(raw[j]));
+    S* p = (S*)&raw[j];
+    float e[V];
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      e[u] = fast_exp(elem<T>::to_float(p[u]) - mx);
+      if constexpr (elem<T>::code == NT_DTYPE_F32) p[u] = e[u];
+    }
+#pragma unroll
+    for (int w = V / 2; w > 0; w /= 2)
+#pragma unroll
+      for (int u = 0; u < w; ++u) e[u] += e[u + w];
+    part[j & 1] += e[0];
+  }
+  const float inv = 1.0f / block_sum<NT / 64>(part[0] + part[1], red);
+  if (t < head) yr[t] = elem<T>::from_float(he * inv);
+  if (t < tail) yb[nvec * V + t] = elem<T>::from_float(te * inv);
+#pragma unroll
+  for (int j = 0; j < R; ++j) {
+    const int i = j * NT + t;
+    u32x4 o;
+    S* q = (S*)&o;
+    if constexpr (ANEW) asm volatile("" : "+v"(raw[j]));
+    const S* p = (const S*)&raw[j];
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      if constexpr (elem<T>::code == NT_DTYPE_F32)
+        q[u] = p[u] * inv;
+      else
+        q[u] = elem<T>::from_float(fast_exp(elem<T>::to_float(p[u]) - mx) * inv);
+    }
+    if (i < nvec) __builtin_nontemporal_store(o, (u32x4*)(yb + (int64_t)i * V));
+  }
+}
+
 // Any strides and any pair of element types (the reference passes strides to its kernel and
 // its store casts to the output's type): one 256-lane workgroup per segment, element-wise
 // loads at the column stride, U elements per lane in flight, an online (max, sum) sweep,
@@ -363,10 +456,11 @@ static void softmax_any_launch(const void* x, int64_t xs, int64_t xcs, void* y, 
 
 // config: 0 = the lane-group kernel for segments of at most 4 vectors per lane of a wave,
 // else the four-wave register path when the segment fits it (16 vectors of 16 bytes per
-// lane at most), else the two-sweep kernel; 1 = four-wave register path; 2 = eight-wave
+// lane at most) and is aligned, else the held kernel (x and y in one 16-byte phase, 256 KiB
+// at most), else the register path element by element, else the two-sweep kernel; 1 = four-wave register path; 2 = eight-wave
 // register path; 3 = one-wave register path; 4 = two-sweep kernel; 5 = lane-group kernel
 // 6 = the any-strides kernel (the only one for a column stride other than 1, so config 0
-// takes it then) (the reference's auto-tuner times num_warps 4, 8, 1:
+// takes it then); 7 and 8 = the held kernel of 256 or 1024 lanes (the reference's auto-tuner times num_warps 4, 8, 1:
 // src/ninetoothed/backends/triton.py:151-155).  A forced kernel whose conditions do not
 // hold returns NT_ERR_INVALID unlaunched.
 template <typename T>
@@ -374,7 +468,7 @@ static int softmax_launch(const void* x, int64_t xs, int64_t xcs, void* y, int64
                           int64_t cols, int64_t block, hipStream_t stream, int config = 0) {
   typedef typename elem<T>::storage S;
   constexpr int V = 16 / sizeof(S);
-  if (config < 0 || config > 6) return NT_ERR_INVALID;
+  if (config < 0 || config > 8) return NT_ERR_INVALID;
   if (rows < 0 || cols < 0 || block <= 0) return NT_ERR_INVALID;
   if (rows == 0 || cols == 0) return 0;
   if (!x || !y) return NT_ERR_INVALID;
@@ -460,16 +554,42 @@ static int softmax_launch(const void* x, int64_t xs, int64_t xcs, void* y, int64
                          ys, cols, block, segs_per_row);
     }
   };
+  // The held kernel with NT lanes and the smallest R that holds the segment at any phase.
+  auto hold = [&](auto nt_c) {
+    constexpr int NT = decltype(nt_c)::value;
+    bool done = false;
+    static_for<1, 5>([&](auto e_c) {
+      constexpr int R = 1 << decltype(e_c)::value;
+      if (done || !coal || len > (int64_t)NT * V * R) return;
+      hipLaunchKernelGGL((softmax_hold_kernel<T, NT, R>), grid, dim3(NT), 0, stream, xp, xs, yp, ys, cols, block,
+                         segs_per_row);
+      done = true;
+    });
+    return done;
+  };
+  using W16 = std::integral_constant<int, 1024>;
   using W4 = std::integral_constant<int, 256>;
   using W8 = std::integral_constant<int, 512>;
   using W1 = std::integral_constant<int, 64>;
   if (config == 0) {
-    if (len > (int64_t)4 * 64 * V || !groups())
-      if (!reg(W4{})) sweep();
+    if (len > (int64_t)4 * 64 * V || !groups()) {
+      // Aligned segments take the register path (fp16 [8192, 8192] 40.9 us, held 40.6); others
+      // in one phase, and those too long for it, are held.  1024 lanes pay for segments of
+      // more than four vectors per lane of 256 where segments leave CUs idle (bf16 [32, 9999]
+      // 5.9 -> 5.1 us; [300, 3001] 4.4 -> 7.0), for aligned ones where the conversions bound
+      // a lane (fp16 [32, 32768] 7.2 -> 5.4; fp32 [64, 16384] 4.9 against 5.0).
+      const bool few = segs < 512;
+      if (vec && len <= (int64_t)16 * 256 * V && !(few && sizeof(S) == 2 && len > (int64_t)8 * 256 * V))
+        reg(W4{});
+      else if (!(few && len > (int64_t)4 * 256 * V ? hold(W16{}) : hold(W4{}) || hold(W16{})) && !reg(W4{}))
+        sweep();
+    }
   } else if (config == 4) {
     sweep();
   } else if (config == 5) {
     if (!groups()) return NT_ERR_INVALID;
+  } else if (config == 7 || config == 8) {
+    if (!(config == 7 ? hold(W4{}) : hold(W16{}))) return NT_ERR_INVALID;
   } else if ((config == 1 && !reg(W4{})) || (config == 2 && !reg(W8{})) || (config == 3 && !reg(W1{}))) {
     return NT_ERR_INVALID;
   }

@@ -1383,6 +1383,37 @@ def test_softmax_configs(config, dtype, cols, block):
         assert torch.allclose(y.float(), ref, atol=tol, rtol=tol)
 
 
+# The held kernel at the edges of what its lanes hold (R vectors of 16 bytes per lane: 16384,
+# 65536 fp32 elements at 16 vectors of 256, 1024 lanes, twice that in 16 bits), rows whose
+# phase changes, short last segments, rows of -inf and a row of nothing else.
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16, torch.float32))
+@pytest.mark.parametrize("config, cols, block", ((7, 1, None), (7, 2049, None), (7, 16383, None), (7, 16384, None),
+                                                 (7, 5000, 1777), (8, 3, None), (8, 16385, None), (8, 65535, None),
+                                                 (8, 65536, None), (8, 70001, 33333), (0, 16385, None), (0, 50257, None),
+                                                 (0, 65537, None), (0, 9999, 4099)))
+def test_softmax_held(config, cols, block, dtype):
+    rows = 6
+    flat = _randn((rows * cols + 3,), dtype, 17, scale=2.0)
+    for offset in (0, 1, 3):
+        x = flat[offset:offset + rows * cols].view(rows, cols)
+        buf = torch.full((rows * cols + 16,), 7.0, dtype=dtype, device=DEV)
+        y = buf[offset % 3:offset % 3 + rows * cols].view(rows, cols)
+        if offset == 3:  # masked elements, a row of nothing else
+            x = x.clone()
+            x[1, ::3] = float("-inf")
+            x[2] = float("-inf")
+        kernels.softmax(x, y, block=block, config=config)
+        blk = cols if block is None else block
+        for c0 in range(0, cols, blk):
+            ref = torch.softmax(x[:, c0:c0 + blk].double(), dim=-1)
+            # one rounding of the result; fp32: exp2 of an argument up to 20 rounded to 2^-24 of it
+            tol = {torch.float16: 2.0**-10, torch.bfloat16: 2.0**-7, torch.float32: 1e-5}[dtype]
+            floor = 2.0**-24 if dtype == torch.float16 else 1e-30
+            assert torch.allclose(y[:, c0:c0 + blk].double(), ref, atol=floor, rtol=tol, equal_nan=True)
+        end = offset % 3 + rows * cols
+        assert (buf[end:] == 7).all() and (buf[:offset % 3] == 7).all()
+
+
 @pytest.mark.parametrize("dtype", (torch.float16, torch.float32))
 @pytest.mark.parametrize("rows, cols, block", ((3000, 128, None), (777, 24, None), (9, 300000, None),
                                                (700, 6000, 2000), (2, 1 << 20, None), (600, 40000, None)))
