@@ -1186,6 +1186,78 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(GemmArgs g) {
   }
 }
 
+// At most 16 rows against more column blocks than CUs: as gemm_skinny_kernel with one block of
+// 16 x 16 and sixteen waves, but one workgroup per CU walks the column blocks.  With a workgroup
+// per block each CU paid the launch, the first loads' latency and the final sum once per block,
+// and read a again for every block (as many bytes through L2 as b).  Here each wave keeps its
+// slice of a in registers (CH 64-deep chunks: 32 VGPRs at K = 4096, which bounds K) and issues
+// the next block's loads of b behind each chunk's MFMAs, so they stay in flight over the sum.
+// Buffer loads bound b by its last row and give zeros past K and past the last block.  Bound by
+// streaming b: bf16 16 x 11008 x 4096 26.1 -> 19.3 us (4.7 TB/s).
+template <typename T, int CH>
+__global__ __launch_bounds__(1024) void gemm_skinny_walk_kernel(GemmArgs g, int blocks) {
+  constexpr int NW = 16;
+  constexpr uint32_t OUTSIDE = 0x80000000u;  // past any bound the launcher allows
+  __shared__ float part[2][NW * 256];
+  const int tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, kg = (lane >> 4) * 8;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int K = (int)g.K, M = (int)g.M;
+  uint32_t bofs[CH][2];
+  u32x4 fa[CH][2], fb[CH][2];
+  const auto ra = __builtin_amdgcn_make_buffer_rsrc((void*)g.a, 0, (int)(((M - 1) * g.sa_m + K) * 2), 0x00020000);
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int k = (wave + c * NW) * skinny::KC + 32 * h + kg;
+      bofs[c][h] = k < K ? (uint32_t)(r16 * g.sb_n + k) * 2 : OUTSIDE;
+      fa[c][h] = __builtin_amdgcn_raw_buffer_load_b128(
+          ra, k < K && r16 < M ? (uint32_t)(r16 * g.sa_m + k) * 2 : OUTSIDE, 0, 0);
+    }
+  auto bounded = [&](int nb) {
+    const int64_t n0 = (int64_t)(nb < blocks ? nb : 0) * 16, left = g.N - n0, rows = left < 16 ? left : 16;
+    return __builtin_amdgcn_make_buffer_rsrc((void*)((const uint16_t*)g.b + n0 * g.sb_n), 0,
+                                             nb < blocks ? (int)(((rows - 1) * g.sb_n + K) * 2) : 0, 0x00020000);
+  };
+  {
+    const auto rb = bounded((int)blockIdx.x);
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) fb[c][h] = __builtin_amdgcn_raw_buffer_load_b128(rb, bofs[c][h], 0, 0);
+  }
+  int buf = 0;
+  for (int nb = (int)blockIdx.x; nb < blocks; nb += (int)gridDim.x, buf ^= 1) {
+    const auto rb = bounded(nb + (int)gridDim.x);
+    floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        acc = skinny::mma16<T>::mma(fa[c][h], fb[c][h], acc);
+        fb[c][h] = __builtin_amdgcn_raw_buffer_load_b128(rb, bofs[c][h], 0, 0);
+      }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) part[buf][(wave * 4 + r) * 64 + lane] = acc[r];
+    // One barrier a block: the sums of this half are read before the next block's barrier,
+    // and written again only after it.  LDS alone is ordered, so b's loads stay in flight.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    if (tid < 256) {
+      float v = 0.0f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) v += part[buf][w * 256 + tid];
+      const int64_t row = 4 * (lane >> 4) + (tid >> 6), col = (int64_t)nb * 16 + r16;
+      if (row < g.M && col < g.N) {
+        float out = g.alpha * round_through(v, g.round_dtype);
+        if (g.c) out += g.beta * load_c<false>(g, row * g.sc_m + col * g.sc_n);
+        store_from_float(g.out, row * g.so_m + col * g.so_n, g.out_dtype, out);
+      }
+    }
+  }
+}
+
 // ----------------------------------------------------------------------------- fp32
 constexpr int F32_TM = 32, F32_TN = 32, F32_KC = 256;
 constexpr int F32_AS = F32_KC + 4;  // a chunk row stride (floats): 16-byte aligned rows
@@ -1783,7 +1855,25 @@ static int gemm16_launch(GemmArgs g, hipStream_t stream, int config = 0, void* w
     using C4 = std::integral_constant<int, 4>;
     using C8 = std::integral_constant<int, 8>;
     using C16 = std::integral_constant<int, 16>;
-    if (g.M <= 16)
+    // One workgroup per CU walking the column blocks, where there are more of those than CUs,
+    // a wave's slice of a fits (K <= 4096) and rows are whole aligned vectors.  bf16 us, this /
+    // a workgroup per block: 16 x 11008 x 4096 19.3 / 26.1, 16 x 4112 x 4096 13.1 / 17.0,
+    // 16 x 8192 x 2048 9.0 / 12.7, 8 x 6000 x 3000 11.7 / 12.9, 7 x 10007 x 1032 6.9 / 7.8,
+    // 1 x 11008 x 4096 17.7 / 18.7, 3 x 7000 x 3400 12.7 / 13.1.  Rows of a that fewer lanes
+    // share gain less, and a second turn of few blocks costs: 1 x 4500 x 2560 9.5 / 9.2.  At
+    // K <= 1024 a wave would hold one chunk in flight.
+    const int64_t col_blocks = cdiv(g.N, 16);
+    auto walk = [&](auto ch_c) {
+      hipLaunchKernelGGL((gemm_skinny_walk_kernel<T, decltype(ch_c)::value>), dim3(256), dim3(1024), 0, stream, g,
+                         (int)col_blocks);
+    };
+    if (g.M <= 16 && skinny_forced && col_blocks > (g.M > 4 ? 256 : 384) && g.K > 1024 && g.K <= 4096 && col_blocks < (1 << 27) &&
+        g.sa_m <= (1 << 25) && g.sb_n <= (1 << 25)) {
+      if (g.K <= 2048)
+        walk(C2{});
+      else
+        walk(C4{});
+    } else if (g.M <= 16)
       go(C1{}, C1{}, C16{}, C4{});
     else if (g.M > 32 && cdiv(g.N, 64) >= 128)
       go(C4{}, C4{}, C8{}, C1{});

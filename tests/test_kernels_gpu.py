@@ -463,6 +463,32 @@ def test_gemm_few_rows_unaligned(mnk, dtype):
 
 
 @pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("mnk", ((16, 4097, 1032), (5, 4112, 2048), (1, 6160, 2056), (16, 11008, 4096), (13, 8200, 4088),
+                                 (4, 6145, 3000), (16, 12289, 1544)))
+def test_gemm_few_rows_walking_columns(mnk, dtype):
+    # One workgroup per CU walking more column blocks than CUs: ragged last blocks, K no
+    # multiple of a wave's share, strided rows followed by infinities, which no product may see.
+    m, n, k = mnk
+    abuf = torch.full((m, k + 8), float("inf"), dtype=dtype, device=DEV)
+    wbuf = torch.full((n, k + 16), float("inf"), dtype=dtype, device=DEV)
+    a, w = abuf[:, :k], wbuf[:, 8:k + 8]
+    a.copy_(_randn((m, k), dtype, 119, 1.0 / math.sqrt(k)))
+    w.copy_(_randn((n, k), dtype, 120))
+    c = _randn((m, n), dtype, 121)
+    obuf = torch.full((m + 1, n + 3), 7.0, dtype=dtype, device=DEV)
+    out = obuf[:m, :n]
+    ref = a.double() @ w.double().t().contiguous()
+    tol = 1e-2 if dtype == torch.bfloat16 else 2e-3  # the result's rounding at magnitudes up to about 4
+    for _ in range(3):  # the same workgroups' LDS halves again
+        kernels.gemm(a, w.t(), out, c=c, alpha=0.5, beta=2.0)
+        assert torch.allclose(out.double(), 0.5 * ref + 2.0 * c.double(), atol=tol, rtol=tol)
+    assert torch.all(obuf[:, n:] == 7.0) and torch.all(obuf[m:] == 7.0)
+    out32 = torch.empty((m, n), dtype=torch.float32, device=DEV)
+    kernels.gemm(a, w.t(), out32)
+    assert torch.allclose(out32.double(), ref, atol=1e-4, rtol=1e-4)
+
+
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
 @pytest.mark.parametrize("bt", (False, True))
 @pytest.mark.parametrize("mnk", (
     (65, 128, 2048), (128, 130, 4096), (200, 264, 2080), (100, 72, 5000),  # split reductions, ragged last split
