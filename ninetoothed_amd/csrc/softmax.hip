@@ -576,10 +576,12 @@ static int softmax_launch(const void* x, int64_t xs, int64_t xcs, void* y, int64
       // Aligned segments take the register path (fp16 [8192, 8192] 40.9 us, held 40.6); others
       // in one phase, and those too long for it, are held.  1024 lanes pay for segments of
       // more than four vectors per lane of 256 where segments leave CUs idle (bf16 [32, 9999]
-      // 5.9 -> 5.1 us; [300, 3001] 4.4 -> 7.0), for aligned ones where the conversions bound
-      // a lane (fp16 [32, 32768] 7.2 -> 5.4; fp32 [64, 16384] 4.9 against 5.0).
+      // 5.9 -> 5.1 us; [300, 3001] 4.4 -> 7.0).  Aligned 16-bit segments of more than eight
+      // vectors a lane are held too: widened, they are 128 registers a lane of the register
+      // path (fp16 [32, 32768] 7.2 -> 5.4, [2048, 32768] 47.3 -> 41.3; fp32 [64, 16384] 4.9
+      // against 5.0).
       const bool few = segs < 512;
-      if (vec && len <= (int64_t)16 * 256 * V && !(few && sizeof(S) == 2 && len > (int64_t)8 * 256 * V))
+      if (vec && len <= (int64_t)(sizeof(S) == 2 ? 8 : 16) * 256 * V)
         reg(W4{});
       else if (!(few && len > (int64_t)4 * 256 * V ? hold(W16{}) : hold(W4{}) || hold(W16{})) && !reg(W4{}))
         sweep();

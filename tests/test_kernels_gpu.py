@@ -1440,6 +1440,18 @@ def test_softmax_held(config, cols, block, dtype):
         assert (buf[end:] == 7).all() and (buf[:offset % 3] == 7).all()
 
 
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("cols", (16384, 16392, 20001, 32760, 32768))
+def test_softmax_held_16_bit_many_rows(cols, dtype):
+    # 512 rows on both sides of eight vectors per lane of 256, aligned and not, up to all sixteen.
+    x = _randn((512, cols), dtype, 18, scale=2.0)
+    y = torch.empty_like(x)
+    kernels.softmax(x, y)
+    tol = 2.0**-10 if dtype == torch.float16 else 2.0**-7  # one rounding of the result
+    floor = 2.0**-24 if dtype == torch.float16 else 1e-30
+    assert torch.allclose(y.double(), torch.softmax(x.double(), dim=-1), atol=floor, rtol=tol)
+
+
 @pytest.mark.parametrize("dtype", (torch.float16, torch.float32))
 @pytest.mark.parametrize("rows, cols, block", ((3000, 128, None), (777, 24, None), (9, 300000, None),
                                                (700, 6000, 2000), (2, 1 << 20, None), (600, 40000, None)))
