@@ -455,9 +455,9 @@ static void softmax_any_launch(const void* x, int64_t xs, int64_t xcs, void* y, 
 }
 
 // config: 0 = the lane-group kernel for segments of at most 4 vectors per lane of a wave,
-// else the four-wave register path when the segment fits it (16 vectors of 16 bytes per
-// lane at most) and is aligned, else the held kernel (x and y in one 16-byte phase, 256 KiB
-// at most), else the register path element by element, else the two-sweep kernel; 1 = four-wave register path; 2 = eight-wave
+// else the held kernel (x and y in one 16-byte phase, 256 KiB at most), else the four-wave
+// register path element by element (8 vectors of 16 bytes per lane at most), else the
+// two-sweep kernel; 1 = four-wave register path; 2 = eight-wave
 // register path; 3 = one-wave register path; 4 = two-sweep kernel; 5 = lane-group kernel
 // 6 = the any-strides kernel (the only one for a column stride other than 1, so config 0
 // takes it then); 7 and 8 = the held kernel of 256 or 1024 lanes (the reference's auto-tuner times num_warps 4, 8, 1:
@@ -573,17 +573,14 @@ static int softmax_launch(const void* x, int64_t xs, int64_t xcs, void* y, int64
   using W1 = std::integral_constant<int, 64>;
   if (config == 0) {
     if (len > (int64_t)4 * 64 * V || !groups()) {
-      // Aligned segments take the register path (fp16 [8192, 8192] 40.9 us, held 40.6); others
-      // in one phase, and those too long for it, are held.  1024 lanes pay for segments of
-      // more than four vectors per lane of 256 where segments leave CUs idle (bf16 [32, 9999]
-      // 5.9 -> 5.1 us; [300, 3001] 4.4 -> 7.0).  Aligned 16-bit segments of more than eight
-      // vectors a lane are held too: widened, they are 128 registers a lane of the register
-      // path (fp16 [32, 32768] 7.2 -> 5.4, [2048, 32768] 47.3 -> 41.3; fp32 [64, 16384] 4.9
-      // against 5.0).
+      // Held by 256 lanes, also where aligned: the register path keeps elements widened and takes
+      // an element-wise branch in a partly filled vector column (fp16 [8192, 5000] 32.4 -> 26.0
+      // us, [8192, 16392] 172 -> 81; fp32 [4096, 12000] 70.6 -> 68.5, equal at [8192, 8192]);
+      // it stays for x and y in different phases.  1024 lanes pay for more than four vectors
+      // per lane of 256 where segments leave CUs idle (bf16 [32, 9999] 5.9 -> 5.1 us, fp16
+      // [32, 32768] 7.2 -> 5.4; [300, 3001] 4.4 -> 7.0).
       const bool few = segs < 512;
-      if (vec && len <= (int64_t)(sizeof(S) == 2 ? 8 : 16) * 256 * V)
-        reg(W4{});
-      else if (!(few && len > (int64_t)4 * 256 * V ? hold(W16{}) : hold(W4{}) || hold(W16{})) && !reg(W4{}))
+      if (!(few && len > (int64_t)4 * 256 * V ? hold(W16{}) : hold(W4{}) || hold(W16{})) && !reg(W4{}))
         sweep();
     }
   } else if (config == 4) {

@@ -138,15 +138,15 @@ def add(lhs, rhs, out):
 
 # --------------------------------------------------------------------- softmax
 # Kernel configurations of the softmax that ``config`` can force (0: the lane-group kernel for
-# segments of at most four 16-byte vectors per lane of a wave, else the four-wave register
-# path for aligned segments it fits, else the held kernel, else the register path element by
-# element, else the two-sweep kernel; the element-wise kernel for a
+# segments of at most four 16-byte vectors per lane of a wave, else the held kernel, else the
+# four-wave register path element by element, else the two-sweep kernel; the element-wise
+# kernel for a
 # column stride other than 1 or an output of another dtype): the register path with
 # workgroups of four, eight or one wave (the reference's num_warps candidates 4, 8, 1), the
 # two-sweep kernel, the lane-group kernel, the element-wise kernel.
 SOFTMAX_CONFIGS = (1, 2, 3, 4, 5, 6)
-# SOFTMAX_FORCED adds the held kernel of 256 and of 1024 lanes, which config 0 takes for
-# unaligned and longer segments and the tuner does not time.
+# SOFTMAX_FORCED adds the held kernel of 256 and of 1024 lanes, which config 0 takes and
+# the tuner does not time.
 SOFTMAX_FORCED = SOFTMAX_CONFIGS + (7, 8)
 SOFTMAX_ANY = 6  # the configuration that takes any strides and any output dtype
 
