@@ -935,18 +935,20 @@ class _TileEmitter(_Emitter):
     def vector_start(self, name, ks, lin):
         """C element number at which the vector of this load starts, where the current loop
         (``self.vec`` consecutive values of ``self.var`` per step, the first ``self.var`` + "0")
-        reads consecutive elements of ``name``; None otherwise."""
+        reads consecutive elements of ``name``; None otherwise.  Records the load in
+        ``self.vectors`` with its head, the element number less the loop variable: a row of a
+        tile of several starts there, and the tensor's limit counts elements of the whole tile."""
         if not self.vec or ks or self.plan.forms.get(name, (0, None))[0] != 1:
             return None
         head, _, last = lin.rpartition(" + ")
         if last != self.var or re.search(rf"\b{self.var}\b", head):
             return None
-        self.vectors.append(name)
+        self.vectors.append((name, head))
         return f"{head} + {self.var}0" if head else f"{self.var}0"
 
     def vector_context(self, root, coords, tag, var, width):
         """``context`` for a loop over vectors of ``width``: (lines ahead of the elements, lines
-        per element ``u``, tensors read as vectors)."""
+        per element ``u``, (tensor, head) of each load that reads vectors)."""
         self.vec, self.var, self.pre, self.vectors = width, var, [], []
         try:
             lines = self.context(root, coords, tag)
@@ -1014,7 +1016,7 @@ class _TileEmitter(_Emitter):
             start = self.vector_start(name, ks, lin)
             if start is not None:  # part of a vector loaded ahead of the unrolled elements
                 vec = f"{self.tag}v{len(self.names)}"
-                self.pre.append(f"      const auto {vec} = nt_ldv<{self.vec}>(p_{name} + ({self.plan.index_expr(name, start)}));")
+                self.pre.append(f"      const auto {vec} = nt_ldv<{self.vec}>(p_{name} + ({self.plan.address(name, start)}));")
                 self.define(v, t, f"(({w}){ld.format(f'{vec}.e[u]')})", exact=True)
                 self.masks[id(v)] = frozenset()
                 return
@@ -1673,13 +1675,15 @@ class TilePlan(GenericPlan):
 
     def _vector_bound(self, vectors, extent, width, name):
         """(C statement, C expression) of the number of elements the vector loop covers: whole
-        vectors inside every vector tensor's row."""
-        cut = [f"lm_{n}" for n in dict.fromkeys(vectors) if self.forms[n][1]]
+        vectors below the limit of every tensor read (or stored) as vectors.  The limit counts
+        elements of the flattened tile, so a vector that starts past ``head`` has that many fewer
+        left, none in a row past the limit."""
+        cut = [(n, head) for n, head in dict.fromkeys(vectors) if self.forms[n][1]]
         if not cut:
             return "", str(extent // width * width)
         expr = str(extent)
-        for c in cut:
-            expr = f"min({expr}, {c})"
+        for n, head in cut:
+            expr = f"min({expr}, " + (f"max(lm_{n} - (int)({head}), 0))" if head else f"lm_{n})")
         return f"const int {name} = {expr} / {width} * {width};", name
 
     def _staged_stores(self, em):
@@ -1788,7 +1792,7 @@ class TilePlan(GenericPlan):
         width = self._vector_width(em) if vectors and self.forms.get(out, (0, None))[0] == 1 else 0
         if width and n_tile >= width:
             pre, each, read = em.vector_context(v, coords, f"z{out}_", "j", width)
-            bound, first = self._vector_bound(read + [out], n_tile, width, f"n_{out}")
+            bound, first = self._vector_bound(read + [(out, "")], n_tile, width, f"n_{out}")
             lines += [
                 f"    {{  // `{out}`, {width} elements per lane",
                 f"    {bound}",
@@ -1801,7 +1805,7 @@ class TilePlan(GenericPlan):
                 *each,
                 f"      ov.e[u] = {stored()};",
                 "      }",
-                f"      nt_stv(p_{out} + ({self.index_expr(out, 'j0')}), ov);",
+                f"      nt_stv(p_{out} + ({self.address(out, 'j0')}), ov);",
                 "    }",
             ]
         if first != str(n_tile):
@@ -1876,9 +1880,13 @@ class TilePlan(GenericPlan):
     def index_expr(self, name, lin):
         if name not in self.forms:
             return f"t_{name}[pb_{name} + {lin}]"
-        step, cut = self.forms[name]
-        at = f"bs_{name}" if step == 0 else f"bs_{name} + (int)({lin}) * {step}" if step != 1 else f"bs_{name} + (int)({lin})"
-        return f"(({lin}) < lm_{name} ? {at} : -1)" if cut else at
+        at = self.address(name, lin)
+        return f"(({lin}) < lm_{name} ? {at} : -1)" if self.forms[name][1] else at
+
+    def address(self, name, lin):
+        """C element offset of element ``lin`` of a tensor with a row form, below its limit."""
+        step = self.forms[name][0]
+        return f"bs_{name}" if step == 0 else f"bs_{name} + (int)({lin}) * {step}" if step != 1 else f"bs_{name} + (int)({lin})"
 
     def level_index(self, name, ks, inner, em):
         """C index-table entry of element ``inner`` of the level of ``name`` reached by the
