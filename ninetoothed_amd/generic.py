@@ -1420,7 +1420,9 @@ class TilePlan(GenericPlan):
         self.shapes = _shapes(ctx, values, probe.const_value, self.carried_shapes)
         self.outputs = list(stores)
         self.kernel_name = "nt_generic_tile"
-        self.forms = {}  # tensor -> (element step, whether rows are cut short): see _row_form
+        # tensor -> (element step: 1, or None where it is the argument st_<tensor>; whether rows are
+        # cut short): see _row_form
+        self.forms = {}
         self.walked = values
         arranged = self.outputs + sorted(
             {_view_chain(e[1])[0] for e in program.effects if e[0] == "view_store"}
@@ -1472,6 +1474,7 @@ class TilePlan(GenericPlan):
                    for n in self.raw]
         params += [f"{_STORAGE[self.scalar_types[n]][0]} s_{n}" for n in self.scalars]
         params.append("long long programs")
+        params += [f"long long st_{n}" for n in self.index_names if self.forms.get(n, (1, False))[0] != 1]
         return params
 
     def _settle_shapes(self, values, probe):
@@ -1670,7 +1673,8 @@ class TilePlan(GenericPlan):
     def _vector_width(self, em):
         """Elements per vector of a loop over consecutive elements: 16 bytes of the narrowest
         tensor addressed without a table, at most 8; 0 when there is none."""
-        sizes = [_SIZES[_torch_dtype_name(self.ctx.dtypes[n])] for n, (step, _) in self.forms.items() if step == 1]
+        sizes = [_SIZES[_torch_dtype_name(self.ctx.dtypes[n])] for n, (step, _) in self.forms.items()
+                 if step == 1 and self.tile_sizes[n] > 1]
         return min(8, 16 // min(sizes)) if sizes and min(sizes) <= 8 else 0
 
     def _vector_bound(self, vectors, extent, width, name):
@@ -1885,8 +1889,7 @@ class TilePlan(GenericPlan):
 
     def address(self, name, lin):
         """C element offset of element ``lin`` of a tensor with a row form, below its limit."""
-        step = self.forms[name][0]
-        return f"bs_{name}" if step == 0 else f"bs_{name} + (int)({lin}) * {step}" if step != 1 else f"bs_{name} + (int)({lin})"
+        return f"bs_{name} + (int)({lin})" + ("" if self.forms[name][0] == 1 else f" * st_{name}")
 
     def level_index(self, name, ks, inner, em):
         """C index-table entry of element ``inner`` of the level of ``name`` reached by the
@@ -2012,7 +2015,7 @@ class TilePlan(GenericPlan):
         if not whole and not np.array_equal(valid, j[None, :] < limit[:, None]):
             return None
         long = int(np.argmax(limit))
-        step = int(rows[long, 1]) - int(rows[long, 0]) if limit[long] > 1 else 0
+        step = int(rows[long, 1]) - int(rows[long, 0]) if limit[long] > 1 else 1
         base = np.where(limit > 0, rows[:, 0], 0).astype(np.int32)
         expected = base[:, None] + (j.astype(np.int64) * step).astype(np.int32)[None, :]
         if not np.array_equal(rows if whole else np.where(valid, rows, 0), expected if whole else np.where(valid, expected, 0)):
@@ -2076,7 +2079,10 @@ class TilePlan(GenericPlan):
         args += [("tensor", n) for n in self.raw]
         args += [("scalar", n, "int64" if self.scalar_types[n] == "int64" else "float32") for n in self.scalars]
         args.append(("i64", self.programs))
-        shaped = self._shaped({n: (form[0], form[2] is not None) for n, form in forms.items()})
+        # Only a unit step, which vectors need, is part of the source: one source (a compilation of
+        # 230-260 ms on a first call) serves every other stride.
+        args += [("i64", forms[n][0]) for n in self.index_names if n in forms and forms[n][0] != 1]
+        shaped = self._shaped({n: (1 if form[0] == 1 else None, form[2] is not None) for n, form in forms.items()})
         return shaped.source(), min(self.programs, 256 * 64), args
 
     def _shaped(self, forms):

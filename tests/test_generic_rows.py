@@ -178,3 +178,26 @@ def test_cut_rows_on_the_host(rows, cols, tile, kind, dtype, tmp_path):
 @pytest.mark.parametrize("rows, cols, tile", CASES + ((1001, 2048, 8), (333, 333, 5)))
 def test_cut_rows(rows, cols, tile, kind, dtype):
     _check(kind, rows, cols, tile, dtype, "cuda", lambda handle, x, out: handle(x, out, ROWS=tile, WIDTH=cols))
+
+
+def row_sum_application(x, out):
+    out = ntl.sum(ntl.cast(x, ntl.float32))  # noqa: F841
+
+
+def test_one_source_serves_every_stride(tmp_path):
+    # Column tiles of tensors of any width: the element step is an argument of the kernel.  Unit
+    # steps, which vectors need, and tiles of one element (any step) share a second one.
+    handle = ninetoothed.make(lambda x, o: (x.tile((ROWS, 1)).flatten(), o.tile((1,))), row_sum_application,
+                              (Tensor(2), Tensor(1)))
+    sources = {}
+    for width in (100, 101, 102, 128, 200, 333, 1):
+        x = (torch.arange(64 * width) % 7).float().view(64, width)
+        for v in (x, x.t().contiguous().t(), x[:1].expand(64, width)):
+            out = torch.full((width,), 7.0)
+            values = dict(zip(handle._abi["public_args"], (v, out)))
+            plan = handle._kernel.specialize(values, {"ROWS": 64})
+            sources.setdefault(plan.sources_for(values)[0], []).append((v, out, values, plan))
+    assert len(sources) == 2
+    for v, out, values, plan in [calls[i] for calls in sources.values() for i in (0, 1, -1)]:
+        _run_on_host(plan, values, tmp_path)
+        assert torch.equal(out, v.sum(0))
