@@ -1423,6 +1423,7 @@ class TilePlan(GenericPlan):
         # tensor -> (element step: 1, or None where it is the argument st_<tensor>; whether rows are
         # cut short): see _row_form
         self.forms = {}
+        self.wide = True  # whether a single long reduction takes the whole workgroup
         self.walked = values
         arranged = self.outputs + sorted(
             {_view_chain(e[1])[0] for e in program.effects if e[0] == "view_store"}
@@ -1529,6 +1530,9 @@ class TilePlan(GenericPlan):
         else:
             items = self.nest.items(None) + [("store", out) for out in self.stores]
         self.blocks = self._scope_blocks(em, None, items)
+        if self.lds_bytes > LDS_BYTES and self.wide:  # without the LDS that whole-workgroup reductions add
+            self.wide = False
+            return self._emit(values)
         if self.lds_bytes > LDS_BYTES:
             raise LoweringError(f"the reductions and loop-carried values of this program need {self.lds_bytes} bytes "
                                 f"of LDS (at most {LDS_BYTES})")
@@ -1598,8 +1602,9 @@ class TilePlan(GenericPlan):
             return f"acc = {comb.format(a='acc', b=f'({term})')};"
 
         step_scalar = accumulate()
-        # A single long reduction takes the whole workgroup (each wave's result through LDS).
-        block = n_out == 1 and extent >= 256
+        # A single long reduction takes the whole workgroup (each wave's result through LDS, where
+        # there is room).
+        block = self.wide and n_out == 1 and extent >= 256
         lanes = 256 if block else (1 if n_out >= 256 else min(64, 1 << int(np.log2(256 // n_out))))
         lanes = max(1, min(lanes, 1 << int(np.ceil(np.log2(max(extent, 1))))))
         step = 256 // lanes
@@ -1641,6 +1646,7 @@ class TilePlan(GenericPlan):
         head = f"    {{  // {kind} over {'all axes' if axis is None else f'axis {axis}'}: {n_out} x {extent}"
         if block:
             self.decls.append(f"  __shared__ {w} {arr}_w[4];")
+            self.lds_bytes += 4 * size
             total = f"{arr}_w[0]"
             for i in range(1, 4):
                 total = comb.format(a=total, b=f"{arr}_w[{i}]")

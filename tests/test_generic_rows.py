@@ -201,3 +201,17 @@ def test_one_source_serves_every_stride(tmp_path):
     for v, out, values, plan in [calls[i] for calls in sources.values() for i in (0, 1, -1)]:
         _run_on_host(plan, values, tmp_path)
         assert torch.equal(out, v.sum(0))
+
+
+def centred_in_place_application(x):
+    x = x - ntl.sum(x)  # noqa: F841
+
+
+@pytest.mark.parametrize("width, whole_workgroup", ((16379, True), (16380, False), (16383, False)))
+def test_lds_of_a_whole_workgroup_reduction_is_counted(width, whole_workgroup):
+    # The stored tile, the sum and (where they fit beside them) the four waves' sums: 64 KiB at most.
+    handle = ninetoothed.make(lambda x: (x.tile((1, WIDTH)),), centred_in_place_application, (Tensor(2),))
+    plan = handle._kernel.specialize({"x": torch.empty(3, width)}, {"WIDTH": width})
+    declared = sum(4 * int(n) for n in re.findall(r"__shared__ float \w+\[(\d+)\]", "\n".join(plan.decls)))
+    assert declared == plan.lds_bytes <= 64 * 1024
+    assert ("red0_w" in "\n".join(plan.decls)) == whole_workgroup
