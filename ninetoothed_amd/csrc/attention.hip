@@ -1332,14 +1332,17 @@ __global__ __launch_bounds__(ak::NW * 64) void attention_keys_kernel(AttnArgs g)
         for (int r = 0; r < 16; ++r) o[i][r] *= alpha;
       m = m_new;
     }
+    // While every score of this wave is -inf, so is m: p is exp2 of the score itself, zero, and
+    // not of -inf - -inf (the keys a wave starts with may all be masked by infinities).
+    const float shift = m == -INFINITY ? 0.f : m;
     frag pf[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       u32x4 w;
 #pragma unroll
       for (int sl = 0; sl < 4; ++sl) {
-        const float p0 = __builtin_amdgcn_exp2f(s[8 * t + 2 * sl] - m);
-        const float p1 = __builtin_amdgcn_exp2f(s[8 * t + 2 * sl + 1] - m);
+        const float p0 = __builtin_amdgcn_exp2f(s[8 * t + 2 * sl] - shift);
+        const float p1 = __builtin_amdgcn_exp2f(s[8 * t + 2 * sl + 1] - shift);
         l += p0 + p1;
         w[sl] = attn::pack2<T>(p0, p1);
       }

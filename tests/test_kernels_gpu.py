@@ -1362,6 +1362,25 @@ def test_attention_few_queries(b, h, sq, sk, d, dtype):
     assert torch.allclose(o.double(), _attention_ref64(q, k, v, False, qs), atol=tol, rtol=tol)
 
 
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("valid", (1, 40, 1500))
+@pytest.mark.parametrize("b, h, sq, sk, d", ((2, 3, 1, 300, 64), (1, 2, 5, 4100, 128), (1, 1, 33, 2048, 128)))
+def test_attention_few_queries_scores_of_minus_infinity(b, h, sq, sk, d, valid, dtype):
+    # Keys masked through a value of -inf in one of their dims: whole tiles, waves and splits
+    # see no finite score, and add nothing.
+    q, k, v = (_randn((b, h, n, d), torch.float32, 124 + i) for i, n in enumerate((sq, sk, sk)))
+    q[..., 0] = 1.0
+    k[..., valid:, 0] = float("-inf")
+    q, k, v = q.to(dtype), k.to(dtype), v.to(dtype)
+    qs = kernels.LOG2E / math.sqrt(d)
+    ref = _attention_ref64(q, k[..., :valid, :], v[..., :valid, :], False, qs)
+    tol = 1e-2 if dtype == torch.float16 else 2e-2
+    for config in (0, 4):
+        o = torch.full_like(q, 7.0)
+        kernels.attention(q, k, v, o, q_scale=qs, config=config)
+        assert torch.allclose(o.double(), ref, atol=tol, rtol=tol)
+
+
 def test_attention_config_conditions_are_checked():
     from ninetoothed_amd.errors import KernelLaunchError
 
