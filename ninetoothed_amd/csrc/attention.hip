@@ -1475,16 +1475,30 @@ static int attention_empty_keys(void* o, const int64_t* os, int o_dtype, int64_t
   return launch_status();
 }
 
-// attention_keys_kernel or attention_fast_kernel, measured fp16/bf16 with K and V rotated past
+// attention_keys_kernel or the kernels below it, measured fp16/bf16 with K and V rotated past
 // the caches.  A workgroup of the first takes 32 queries through 4,096 keys of D = 128 in about
-// 57 us, one of the second 256 queries in 107, so the first is the faster while one round of
-// its workgroups fits the chip or one block holds all the queries of a head (keys / fast us:
-// [8,32,1,4000,128] 93 / 150, [1,32,1,4096,128] 24 / 106, [4,32,64,4096,128] 57 / 108,
-// [32,32,32,4096,128] 369 / 441, [1,8,1024,1024,128] 17.4 / 32.6, [2,8,128,128,64] 6.2 / 12.7);
-// two blocks a head beat the four-wave kernel, too ([16,32,64,4096,128] 211 / 232).
-static bool attention_keys_wanted(int64_t BH, int64_t Sq) {
+// 57 us, one of attention_fast_kernel 256 queries in 107, so the first is the faster while one
+// round of its workgroups fits the chip or one block holds all the queries of a head (keys /
+// before us: [8,32,1,4000,128] 93 / 150, [1,32,1,4096,128] 24 / 106, [4,32,64,4096,128] 57 / 108,
+// [32,32,32,4096,128] 369 / 441, [1,8,1024,1024,128] 17.4 / 32.6, [2,8,128,128,64] 6.2 / 12.7),
+// and for two blocks of very many heads ([16,32,64,4096,128] 211 / 232).
+// Each of its waves pays for merging its state, however few its keys, and with causal masking
+// the kernels below it take 64-key tiles: few keys a query stay with them, up to a line that
+// lies higher where the heads alone fill the chip (us, this / before; the lines hold for both
+// types, fp16 crossing later).  One block, D = 128: bf16 32 queries of 64 heads over 64 keys
+// 10.3 / 8.8, 128 11.6 / 11.0; of 4,096 heads over 128 185 / 171; fp16 16 of 2,048 heads over 192
+// 80 / 69, 224 84.5 / 83; 32 over 224 104 / 90.  D = 64, 32 of 64 heads over 64 keys 7.2 / 6.7,
+// of 512 11.7 / 13.3.  More blocks within one round: D = 128 64 of 64 heads over 64 keys 10.5 /
+// 9.0, 192 13.6 / 13.6; D = 64 over 64 7.2 / 6.5, 96 7.6 / 8.0.  Two blocks of 512 heads, fp16:
+// D = 128 over 3,072 keys 173 / 167, 4,096 215 / 220; D = 64 over 512 23.6 / 22.8; causal,
+// never (D = 128 27 / 16).
+static bool attention_keys_wanted(int64_t BH, int64_t Sq, int64_t Sk, int64_t D, bool causal) {
   const int64_t nq = cdiv(Sq, ak::BQ);
-  return nq == 1 || nq * BH <= 256 || (nq == 2 && BH >= 512);
+  const bool wide = D > 64;
+  if (nq == 1 && wide) return Sk >= (BH < 512 ? (causal ? 4 : 6) : (causal ? 8 : 16)) * Sq;
+  if (nq == 1) return BH >= 512 || Sk > 2 * Sq;
+  if (nq * BH <= 256) return Sk >= (wide && !causal ? 192 : 96);
+  return nq == 2 && BH >= 512 && !causal && Sk >= (wide ? 4096 : 768);
 }
 // Workgroups per query block: as many as fill the 256 CUs once, each with at least 32 tiles
 // (1,024 keys), at most 8: splits cost the merge launch (us at 1 / 2 / 4 / 8 / 16 splits:
@@ -1550,7 +1564,7 @@ static int attention_launch(const void* q, const int64_t* qs, const void* k, con
   const bool fast_fits = fast_ok(dm), pipe_fits = D == 128 && fast_fits;
   const bool keys_fits = fast_fits && B * H <= 0x7fffffffLL / 64;
   if ((config == 1 && !pipe_fits) || (config == 2 && !fast_fits) || (config == 4 && !keys_fits)) return NT_ERR_INVALID;
-  if (config == 4 || (config == 0 && keys_fits && attention_keys_wanted(B * H, Sq))) {
+  if (config == 4 || (config == 0 && keys_fits && attention_keys_wanted(B * H, Sq, Sk, D, causal != 0))) {
     const int64_t qblocks = cdiv(Sq, ak::BQ);
     // a causal block sees only the keys up to its queries: never split
     int splits = config == 0 && !causal ? attention_splits(B * H, Sq, Sk) : 1;
@@ -1811,7 +1825,7 @@ extern "C" int64_t nt_attention_workspace_size(int64_t B, int64_t H, int64_t Sq,
                                                int dtype) {
   if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || D <= 0 || D > 128 || causal) return 0;
   if (dtype != NT_DTYPE_F16 && dtype != NT_DTYPE_BF16) return 0;
-  if (!nt::attention_keys_wanted(B * H, Sq)) return 0;
+  if (!nt::attention_keys_wanted(B * H, Sq, Sk, D, false)) return 0;
   return nt::attention_workspace(B * H, Sq, Sk, D, nt::attention_splits(B * H, Sq, Sk));
 }
 extern "C" int nt_attention_ws_f16(NT_ATTN_PARAMS, void* workspace, int64_t workspace_bytes) {
