@@ -1732,9 +1732,16 @@ static int conv_launch(const void* x, const int64_t* xs, const void* w, const in
   // Its output as 16-byte runs of 8 positions of one channel, or else element by element.
   g.qvec = Q % 8 == 0 && ys[3] == 1 && ys[0] % 8 == 0 && ys[1] % 8 == 0 && ys[2] % 8 == 0 && (uintptr_t)y % 16 == 0;
   g.Mp = cdiv(g.M, 8) * 8;
+  // Input rows of whole aligned 16-byte chunks: the re-layout kernels that read them as such.
+  const bool fast_relayout = xs[3] == 1 && W % 8 == 0 && (uintptr_t)x % 16 == 0 && (xs[0] * 2) % 16 == 0 &&
+                             (xs[1] * 2) % 16 == 0 && (xs[2] * 2) % 16 == 0;
   // The im2col path: a filter dense over (c, r, s) in place, whole 32-deep k-tiles, the matrix
-  // and the split partials in the workspace.
-  if (config == 8 || (config == 0 && cols_wanted(g.M, K, R, S, Hp, Wp))) {
+  // and the split partials in the workspace.  A few workgroups of larger planes stage them no
+  // faster than conv_relayout_pipe_kernel, where it can run (us, im2col / re-laid: 5 x 5
+  // [1,64,8,8] x 64 16.2 / 14.0, 3 x 3 at stride 2 [1,64,16,16] x 64 14.9 / 13.0, [1,128,16,16] x
+  // 128 15.7 / 14.0, [4,96,16,16] x 256 17.1 / 14.7, [1,512,16,16] x 512 18.8 / 32.9).
+  const bool few_planes = fast_relayout && ((Hp * Wp >= 144 && N * (C / 16) < 16) || (Hp * Wp >= 256 && N * (C / 16) < 32));
+  if (config == 8 || (config == 0 && cols_wanted(g.M, K, R, S, Hp, Wp) && !few_planes)) {
     const int64_t KG = C * R * S, cb = cols_channels(C, Hp, Wp, R * S);
     const int64_t cols_bytes = cdiv(g.M * KG * 2, 256) * 256;
     const bool fits = cb > 0 && R * S > 0 && KG >= 96 && KG % 32 == 0 && ws[3] == 1 && ws[2] == S && ws[1] == R * S &&
@@ -1859,8 +1866,6 @@ static int conv_launch(const void* x, const int64_t* xs, const void* w, const in
     uint16_t* wt = (uint16_t*)((char*)workspace + ((N * Hp * Wp * Cl * 2 + 255) / 256) * 256);
     int64_t fblocks = K * R * S;  // filter rows of the fast re-layout (at most 4096 workgroups)
     if (fblocks > 4096) fblocks = 4096;
-    const bool fast_relayout = xs[3] == 1 && W % 8 == 0 && (uintptr_t)x % 16 == 0 && (xs[0] * 2) % 16 == 0 &&
-                               (xs[1] * 2) % 16 == 0 && (xs[2] * 2) % 16 == 0;
     if (fast_relayout && Cl * W * 2 <= RELAYOUT_STAGE_BYTES && (Cl / 8) * (W / 8) <= 256) {
       // rows in workgroups that each take several, two per CU; the filter one channel k at a time
       const int64_t row_blocks = N * Hp < 512 ? N * Hp : 512, kblocks = K < 256 ? K : 256;
@@ -1877,11 +1882,19 @@ static int conv_launch(const void* x, const int64_t* xs, const void* w, const in
     } else {
       // small planes: 64 channels per workgroup when that still gives every CU one, else 32
       const int64_t cbp = Cl % 64 == 0 && N * (Cl / 64) >= 256 && 64 * Hp * Wp * 2 <= PLANES_LDS ? 64 : 32;
-      const bool planes = Hp * Wp < PLANES_BELOW && cbp * Hp * Wp * 2 <= PLANES_LDS && N * (Cl / cbp) <= 0x3fffffff;
       const bool filter9 = dma && R == 3 && S == 3 && Cl == C && ws[3] == 1 && ws[2] == 3 && ws[1] == 9 &&
                            ws[0] == C * 9 && (uintptr_t)w % 16 == 0 && K * (C / 32) <= 0x3fffffff;
+      // Where the filter needs a launch of its own all the same, a workgroup's trip through its
+      // planes (whose length goes with their positions) has to be hidden behind others: us,
+      // conv_planes_kernel / nchw_to_nhwc_pad_kernel, 1 x 1 filters: [1,32,18,18] x 32 20.8 /
+      // 16.0, [4,64,14,14] x 64 20.2 / 18.1, [16,128,14,14] x 128 21.1 / 22.0, [1,64,7,7] x 64 13.3 /
+      // 14.9, [64,64,18,18] x 64 24.7 / 29.0 (2 x 2: 25.6 / 24.6).
+      const int64_t plane_blocks = N * (Cl / cbp);
+      const bool planes = Hp * Wp < PLANES_BELOW && cbp * Hp * Wp * 2 <= PLANES_LDS && plane_blocks <= 0x3fffffff &&
+                          (filter9 || Hp * Wp < 144 || (Hp * Wp < 256 && plane_blocks >= 64) ||
+                           plane_blocks >= (R * S == 1 ? 128 : 256));
       if (planes) {
-        const int64_t in_blocks = N * (Cl / cbp), units = filter9 ? K * (C / 32) : 0;
+        const int64_t in_blocks = plane_blocks, units = filter9 ? K * (C / 32) : 0;
         const int64_t lds = std::max<int64_t>(cbp * Hp * Wp * 2, 7 * 288 * 2);
         hipLaunchKernelGGL(conv_planes_kernel, dim3((unsigned)(in_blocks + cdiv(units, 7))), dim3(256), (size_t)lds, stream,
                            (const uint16_t*)x, xp, (const uint16_t*)w, wt, g, (int)cbp, (int)Hp, (int)Wp,
