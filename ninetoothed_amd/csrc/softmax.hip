@@ -577,9 +577,10 @@ static int softmax_launch(const void* x, int64_t xs, int64_t xcs, void* y, int64
       // an element-wise branch in a partly filled vector column (fp16 [8192, 5000] 32.4 -> 26.0
       // us, [8192, 16392] 172 -> 81; fp32 [4096, 12000] 70.6 -> 68.5, equal at [8192, 8192]);
       // it stays for x and y in different phases.  1024 lanes pay for more than four vectors
-      // per lane of 256 where segments leave CUs idle (bf16 [32, 9999] 5.9 -> 5.1 us, fp16
-      // [32, 32768] 7.2 -> 5.4; [300, 3001] 4.4 -> 7.0).
-      const bool few = segs < 512;
+      // per lane of 256 while there is a CU for each segment (bf16 [32, 9999] 5.9 -> 5.1 us, fp16
+      // [32, 32768] 7.2 -> 5.4; [300, 3001] 4.4 -> 7.0; with two on a CU fp16 [300, 32768] 13.4
+      // against 10.2 on 256 lanes, [511, 32768] 15.8 against 11.5, fp32 [384, 16384] 9.5 / 9.2).
+      const bool few = segs <= 256;
       if (!(few && len > (int64_t)4 * 256 * V ? hold(W16{}) : hold(W4{}) || hold(W16{})) && !reg(W4{}))
         sweep();
     }
