@@ -1150,11 +1150,14 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(GemmArgs g) {
       const int64_t left = g.K - (k_tail + 32 * h + kg);  // k of this lane inside K
       auto partial = [&](const uint16_t* row) {
         const uint16_t* p = row + k_tail + 32 * h;
-        if (left >= 8) return ((const skinny::unaligned16*)p)->v;
         u32x4 v = {0u, 0u, 0u, 0u};
+        if (left >= 8) {
+          v = ((const skinny::unaligned16*)p)->v;
+        } else if (left > 0) {  // (its own branch: K a multiple of 8 jumps over the elements)
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (u < left) v[u >> 1] |= (uint32_t)p[u] << (16 * (u & 1));
+          for (int u = 0; u < 8; ++u)
+            if (u < left) v[u >> 1] |= (uint32_t)p[u] << (16 * (u & 1));
+        }
         return v;
       };
 #pragma unroll
@@ -1844,7 +1847,12 @@ static int gemm16_launch(GemmArgs g, hipStream_t stream, int config = 0, void* w
   // leaves no fewer workgroups than CUs (32 x 4096 x 4096: 14.3 against 18.4 us with 32 x 32),
   // 32 x 32 blocks from 256 of those (64 x 4096 x 4096: 18.5 against 25.4 with 32 x 16), 64 x 64
   // from 128 column blocks (64 x 11008 x 4096: 34.4 against 50.1 with 32 x 32).
-  if (config == 5 || (config == 0 && skinny)) {
+  // Past 32 rows a workgroup's columns of a long b are too many to read a for again: the
+  // 128-wide tiles, where they can run, from 129 of them (bf16 us, this kernel / those tiles:
+  // 48 x 16384 x 1024 11.8 / 17.9, 48 x 20000 x 1024 20.7 / 17.7, 64 x 32000 x 512 17.1 / 13.3,
+  // 64 x 50000 x 4096 142 / 104, 33 x 32000 x 4096 64.7 / 68.5).
+  const bool long_b = g.M > 32 && ok128 && tiles128 > 128;
+  if (config == 5 || (config == 0 && skinny && !long_b)) {
     auto go = [&](auto mb_c, auto nb_c, auto nw_c, auto d_c) {
       constexpr int MB = decltype(mb_c)::value, NB = decltype(nb_c)::value, NW = decltype(nw_c)::value;
       const dim3 gridS((unsigned)cdiv(g.N, 16 * NB), (unsigned)cdiv(g.M, 16 * MB));
@@ -1873,11 +1881,29 @@ static int gemm16_launch(GemmArgs g, hipStream_t stream, int config = 0, void* w
         walk(C2{});
       else
         walk(C4{});
+    } else if (g.M <= 32 && g.K <= 1024 && g.N > (g.M <= 16 ? 4096 : 8192)) {
+      // Few chunks of K: most of sixteen waves would idle, and a workgroup of 16 columns would be
+      // all launch and final sum.  32 columns on as few waves as the column blocks leave room
+      // for.  bf16 us, this / 16 columns (sixteen waves, or eight past 16 rows): 1 x 16384 x 8
+      // 3.1 / 5.6, 8 x 131072 x 64 7.3 / 28, 16 x 32000 x 256 5.9 / 11.4, 16 x 131072 x 1024
+      // 59 / 85; 32 x 16384 x 256 4.8 / 6.4, 32 x 32000 x 64 4.6 / 7.4, 32 x 131072 x 8 10.9 /
+      // 29.8 (four waves 13.7), 32 x 131072 x 512 37 / 62.
+      if (g.M <= 16) {
+        if (g.N <= 16384)
+          go(C1{}, C2{}, C8{}, C2{});
+        else
+          go(C1{}, C2{}, C4{}, C1{});
+      } else if (g.N <= 16384)
+        go(C2{}, C2{}, C8{}, C2{});
+      else if (g.K <= 128 && g.N > 65536)
+        go(C2{}, C2{}, C2{}, C1{});
+      else
+        go(C2{}, C2{}, C4{}, C1{});
     } else if (g.M <= 16)
       go(C1{}, C1{}, C16{}, C4{});
     else if (g.M > 32 && cdiv(g.N, 64) >= 128)
       go(C4{}, C4{}, C8{}, C1{});
-    else if (g.M > 32 && 2 * cdiv(g.N, 32) >= 256)
+    else if (g.M > 32 && 2 * cdiv(g.N, 32) >= 256 && g.K >= skinny::KC)
       go(C2{}, C2{}, C8{}, C2{});
     else
       go(C2{}, C1{}, C8{}, C4{});

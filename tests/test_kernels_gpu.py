@@ -463,6 +463,29 @@ def test_gemm_few_rows_unaligned(mnk, dtype):
 
 
 @pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
+@pytest.mark.parametrize("mnk", ((1, 4097, 8), (16, 16384, 1024), (5, 16385, 63), (16, 20001, 130), (17, 8193, 1024),
+                                 (32, 16384, 72), (20, 16385, 1000), (32, 65537, 128), (31, 65600, 7), (24, 65537, 129),
+                                 (33, 16384, 104), (64, 16392, 104), (40, 20000, 1000), (64, 4096, 63)))
+def test_gemm_few_rows_of_short_k(mnk, dtype):
+    # Both sides of each line between the tilings of a short K against many columns, and of the
+    # 128-wide tiles past 32 rows; aligned rows and others, infinities past K and N.
+    m, n, k = mnk
+    for shift in (0, 1):
+        abuf = torch.full((m, k + 8 + shift), float("inf"), dtype=dtype, device=DEV)
+        wbuf = torch.full((n, k + 8 + shift), float("inf"), dtype=dtype, device=DEV)
+        a, w = abuf[:, shift:k + shift], wbuf[:, shift:k + shift]
+        a.copy_(_randn((m, k), dtype, 122, 1.0 / math.sqrt(k)))
+        w.copy_(_randn((n, k), dtype, 123))
+        obuf = torch.full((m + 1, n + 8), 7.0, dtype=dtype, device=DEV)
+        out = obuf[:m, :n]
+        kernels.gemm(a, w.t(), out)
+        ref = a.double() @ w.double().t().contiguous()
+        tol = 1e-2 if dtype == torch.bfloat16 else 2e-3  # the result's rounding at magnitudes up to about 4
+        assert torch.allclose(out.double(), ref, atol=tol, rtol=tol)
+        assert torch.all(obuf[:, n:] == 7.0) and torch.all(obuf[m:] == 7.0)
+
+
+@pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
 @pytest.mark.parametrize("mnk", ((16, 4097, 1032), (5, 4112, 2048), (1, 6160, 2056), (16, 11008, 4096), (13, 8200, 4088),
                                  (4, 6145, 3000), (16, 12289, 1544)))
 def test_gemm_few_rows_walking_columns(mnk, dtype):
