@@ -1639,6 +1639,12 @@ __global__ void gemm_k0_kernel(GemmArgs g) {
 // 8192 814 against 770) and loses from 144 (3072^3 681 against 849).
 constexpr int64_t DMA128_BELOW = 136;
 
+// Whether the rows of a row-major b past K that the DMA kernels take (whole 32-deep k-tiles, at
+// least three) lie past its buffer resource, which gives zeros: with rows that overlap (an
+// expanded row, a sliding window) they are elements of b, and a's zeros times an infinity there
+// are not zero.
+static bool b_tail_zero(int64_t K, int64_t sb_k, int64_t N) { return (K % 32 == 0 && K >= 3 * 32) || sb_k >= N; }
+
 // The route of a 16-bit product through a workspace (config 0):
 //   - a reduction split over workgroups, for outputs of few 128 x 128 tiles;
 //   - operands that the DMA kernels cannot read where they are (rows off a 16-byte boundary, K
@@ -1689,7 +1695,7 @@ static bool gemm16_route(const GemmArgs& g, Gemm16Route& r) {
   r.Kp = k_odd ? std::max<int64_t>(96, cdiv(g.K, 8) * 8) : g.K;
   r.Nbp = cdiv(g.N, 8) * 8;
   r.pad_a = k_odd || g.sa_m < 0 || g.sa_m % 8 != 0 || (uintptr_t)g.a % 16 != 0;
-  r.pad_b = (r.bt ? k_odd : g.N % 8 != 0) || sb < 0 || sb % 8 != 0 || (uintptr_t)g.b % 16 != 0;
+  r.pad_b = (r.bt ? k_odd : g.N % 8 != 0 || !b_tail_zero(g.K, sb, g.N)) || sb < 0 || sb % 8 != 0 || (uintptr_t)g.b % 16 != 0;
   const int64_t t256 = cdiv(g.M, GB_M) * cdiv(g.N, GB_N), t128 = cdiv(g.M, 128) * cdiv(g.N, 128);
   if (t128 > 0x7fffffffLL) return false;
   const bool padded = r.pad_a || r.pad_b, fast = gemm16_out_fast(g);
@@ -1807,7 +1813,7 @@ static int gemm16_launch(GemmArgs g, hipStream_t stream, int config = 0, void* w
   // multiples of 8, so that every 16-byte operand chunk lies wholly inside or wholly past
   // the matrix (its buffer resources return zeros past the end, per chunk).
   const bool dma_nn = aligned && g.N % 8 == 0 && g.K % 8 == 0 && (GB_M - 1) * g.sa_m + g.K <= 0x3fffffffLL &&
-                      (g.K - 1) * g.sb_k + GB_N <= 0x3fffffffLL && g.K >= 3 * 32;
+                      (g.K - 1) * g.sb_k + GB_N <= 0x3fffffffLL && g.K >= 3 * 32 && b_tail_zero(g.K, g.sb_k, g.N);
   // ... or with b k-contiguous (b^T rows, as a's): any N.
   const bool dma_bt = g.sa_k == 1 && g.sb_k == 1 && g.sa_m >= 0 && (uintptr_t)g.a % 16 == 0 && (uintptr_t)g.b % 16 == 0 &&
                       (g.sa_m * 2) % 16 == 0 && (g.sb_n * 2) % 16 == 0 && g.sb_n > 0 && g.K % 8 == 0 &&
@@ -1821,7 +1827,7 @@ static int gemm16_launch(GemmArgs g, hipStream_t stream, int config = 0, void* w
                               127 * g.sc_m + 128 <= 0x3fffffffLL);
   // gemm_dma128_kernel: the same conditions on 128 x 128 tiles, with the fast epilogue only.
   const bool dma128_nn = aligned && g.N % 8 == 0 && g.K % 8 == 0 && 127 * g.sa_m + g.K <= 0x3fffffffLL &&
-                         (g.K - 1) * g.sb_k + 128 <= 0x3fffffffLL && g.K >= 3 * 32;
+                         (g.K - 1) * g.sb_k + 128 <= 0x3fffffffLL && g.K >= 3 * 32 && b_tail_zero(g.K, g.sb_k, g.N);
   const bool dma128_bt = g.sa_k == 1 && g.sb_k == 1 && g.sa_m >= 0 && (uintptr_t)g.a % 16 == 0 &&
                          (uintptr_t)g.b % 16 == 0 && (g.sa_m * 2) % 16 == 0 && (g.sb_n * 2) % 16 == 0 && g.sb_n > 0 &&
                          g.K % 8 == 0 && 127 * g.sa_m + g.K <= 0x3fffffffLL && 127 * g.sb_n + g.K <= 0x3fffffffLL &&
@@ -2196,6 +2202,7 @@ int gemm16_batch128(int dtype, const void* a, int64_t sa_m, int64_t sa_b, const 
       sa_b % 8 || sb_b % 8 || so_b % 8)
     return NT_ERR_INVALID;
   if (127 * sa_m + K > 0x3fffffffLL || (K - 1) * sb_k + 128 > 0x3fffffffLL) return NT_ERR_INVALID;
+  if (!b_tail_zero(K, sb_k, N)) return NT_ERR_INVALID;
   const int64_t tiles = cdiv(M, 128) * cdiv(N, 128);
   if (tiles > 0x7fffffffLL) return NT_ERR_INVALID;
   if (check_only) return 0;

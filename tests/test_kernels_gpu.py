@@ -462,6 +462,36 @@ def test_gemm_few_rows_unaligned(mnk, dtype):
     assert torch.allclose(out.double(), ref, atol=tol, rtol=tol)
 
 
+@pytest.mark.parametrize("stride", (0, 8))
+@pytest.mark.parametrize("k", (40, 104, 131, 2056))
+def test_gemm_rows_of_b_that_overlap(k, stride):
+    # A b of one row for every k (an expanded row), or of rows that begin inside one another: what
+    # lies where a row past K would be is a row's value, and an infinity there is not zero.
+    m, n = 100, 200
+    for dtype in (torch.float16, torch.bfloat16):
+        base = _randn((stride * k + n + 8,), dtype, 124, 0.1)
+        base[5::40] = float("inf")
+        b = base.as_strided((k, n), (stride, 1))
+        a = torch.full((m, k), 1.0 / k, dtype=dtype, device=DEV)
+        out = torch.empty((m, n), dtype=dtype, device=DEV)
+        kernels.gemm(a, b, out)
+        ref = (a[:1].double() @ b.double().contiguous()).expand(m, n)
+        # the result's rounding; a's elements all round alike, by up to 2^-9 of the sum in bf16
+        assert torch.allclose(out.double(), ref, atol=1e-2, rtol=1e-2, equal_nan=True)
+
+
+def test_conv2d_channels_that_overlap():
+    # 1 x 1 filters over one channel expanded to 104: the products' rows past the last channel.
+    x = _randn((2, 1, 8, 8), torch.float16, 125)
+    x[0, 0, 3, 3] = float("inf")
+    x = x.expand(2, 104, 8, 8)
+    w = torch.full((64, 104, 1, 1), 1.0 / 104, dtype=torch.float16, device=DEV)
+    y = torch.empty((2, 64, 8, 8), dtype=torch.float16, device=DEV)
+    kernels.conv2d(x, w, y)
+    ref = x[:, :1].double().expand(2, 64, 8, 8) * (104 * w[0, 0, 0, 0].double())
+    assert torch.allclose(y.double(), ref, atol=1e-2, rtol=1e-2)
+
+
 @pytest.mark.parametrize("dtype", (torch.float16, torch.bfloat16))
 @pytest.mark.parametrize("mnk", ((1, 4097, 8), (16, 16384, 1024), (5, 16385, 63), (16, 20001, 130), (17, 8193, 1024),
                                  (32, 16384, 72), (20, 16385, 1000), (32, 65537, 128), (31, 65600, 7), (24, 65537, 129),
