@@ -314,6 +314,17 @@ def check_gemm(a, b, out, c=None, round_dtype=None, config=0):
     return _entry_name("nt_gemm", a.dtype), out_code, rd
 
 
+def _workspace(nbytes, device):
+    """A call's workspace from torch's stream-ordered caching allocator (taken on every call, as
+    conv2d's), or None where memory has run out: the kernels that use one run without it too."""
+    import torch
+
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def bind_gemm(a, b, out, c=None, round_dtype=None, config=0):
     """launch(a, b, out, c, alpha, beta): out = cast(beta * c + alpha * round(a @ b)).
 
@@ -344,21 +355,6 @@ def bind_gemm(a, b, out, c=None, round_dtype=None, config=0):
             for slot, t in zip(_GEMM_POINTER_SLOTS, (a, b, c, out)):
                 sample[slot] = t.data_ptr() if t is not None else 0
             nbytes = int(_lib.load().nt_gemm_workspace_size((ctypes.c_int64 * 22)(*sample)))
-        if nbytes:
-            import torch
-
-            addr_ws = _packed_address("nt_gemm_packed_ws")
-            template_ws = template + struct.pack("<2q", 0, nbytes)
-
-            def launch(a, b, out, c, alpha, beta):
-                # from torch's stream-ordered caching allocator on every call, as conv2d's
-                ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-                code = call(addr_ws, template_ws, _GEMM_WS_POINTER_SLOTS, (a, b, c, out, ws), _GEMM_VALUE_SLOTS,
-                            (_float_bits(alpha), _float_bits(beta), stream() or 0))
-                if code:
-                    _raise(code, name)
-
-            return launch
 
         def launch(a, b, out, c, alpha, beta):
             code = call(addr, template, _GEMM_POINTER_SLOTS, (a, b, c, out), _GEMM_VALUE_SLOTS,
@@ -366,7 +362,21 @@ def bind_gemm(a, b, out, c=None, round_dtype=None, config=0):
             if code:
                 _raise(code, name)
 
-        return launch
+        if not nbytes:
+            return launch
+        addr_ws = _packed_address("nt_gemm_packed_ws")
+        template_ws = template + struct.pack("<2q", 0, nbytes)
+
+        def launch_ws(a, b, out, c, alpha, beta):
+            ws = _workspace(nbytes, device)
+            if ws is None:
+                return launch(a, b, out, c, alpha, beta)
+            code = call(addr_ws, template_ws, _GEMM_WS_POINTER_SLOTS, (a, b, c, out, ws), _GEMM_VALUE_SLOTS,
+                        (_float_bits(alpha), _float_bits(beta), stream() or 0))
+            if code:
+                _raise(code, name)
+
+        return launch_ws
 
     def launch(a, b, out, c, alpha, beta):
         code = fn(a.data_ptr(), sa_m, sa_k, b.data_ptr(), sb_k, sb_n, c.data_ptr() if c is not None else None, sc_m,
@@ -517,27 +527,26 @@ def bind_attention(q, k, v, o, causal=False, q_scale=LOG2E, config=0):
     if not config and _lib.dtype_code(q.dtype) != _lib.DTYPE_F32:
         nbytes = int(_lib.load().nt_attention_workspace_size(bsz, heads, sq, sk, d, 1 if causal else 0,
                                                              _lib.dtype_code(q.dtype)))
-    if nbytes:
-        import torch
-
-        fn, name = _entry(f"nt_attention_ws_{_lib.dtype_suffix(q.dtype)}")
-
-        def launch(q, k, v, o):
-            # from torch's stream-ordered caching allocator on every call, as conv2d's
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-            code = fn(q.data_ptr(), qs, k.data_ptr(), ks, v.data_ptr(), vs, o.data_ptr(), os_, *tail, stream(),
-                      ws.data_ptr(), nbytes)
-            if code:
-                _raise(code, name)
-
-        return launch
 
     def launch(q, k, v, o):
         code = fn(q.data_ptr(), qs, k.data_ptr(), ks, v.data_ptr(), vs, o.data_ptr(), os_, *tail, stream(), *extra)
         if code:
             _raise(code, name)
 
-    return launch
+    if not nbytes:
+        return launch
+    fn_ws, name_ws = _entry(f"nt_attention_ws_{_lib.dtype_suffix(q.dtype)}")
+
+    def launch_ws(q, k, v, o):
+        ws = _workspace(nbytes, device)
+        if ws is None:
+            return launch(q, k, v, o)
+        code = fn_ws(q.data_ptr(), qs, k.data_ptr(), ks, v.data_ptr(), vs, o.data_ptr(), os_, *tail, stream(),
+                     ws.data_ptr(), nbytes)
+        if code:
+            _raise(code, name_ws)
+
+    return launch_ws
 
 
 def attention(q, k, v, o, causal=False, q_scale=LOG2E, config=0):

@@ -462,6 +462,26 @@ def test_gemm_few_rows_unaligned(mnk, dtype):
     assert torch.allclose(out.double(), ref, atol=tol, rtol=tol)
 
 
+def test_workspaces_that_do_not_fit(monkeypatch):
+    # A call that can run without its workspace does so where the allocation fails.
+    a, w = _randn((300, 4099), torch.float16, 126, 1.0 / 64), _randn((4099, 512), torch.float16, 127)
+    q, k, v = (_randn((1, 2, n, 128), torch.float16, 128 + i) for i, n in enumerate((1, 8192, 8192)))
+    out, o = torch.empty((300, 512), dtype=torch.float16, device=DEV), torch.empty_like(q)
+    qs = kernels.LOG2E / math.sqrt(128)
+    product, attend = kernels.bind_gemm(a, w, out), kernels.bind_attention(q, k, v, o, q_scale=qs)
+    ref, att = a.double() @ w.double(), _attention_ref64(q, k, v, False, qs)
+
+    def refused(*args, **kwargs):
+        raise torch.OutOfMemoryError("no memory")
+
+    monkeypatch.setattr(torch, "empty", refused)
+    product(a, w, out, None, 1.0, 0.0)
+    attend(q, k, v, o)
+    monkeypatch.undo()
+    assert torch.allclose(out.double(), ref, atol=2e-3, rtol=2e-3)
+    assert torch.allclose(o.double(), att, atol=1e-2, rtol=1e-2)
+
+
 @pytest.mark.parametrize("stride", (0, 8))
 @pytest.mark.parametrize("k", (40, 104, 131, 2056))
 def test_gemm_rows_of_b_that_overlap(k, stride):
