@@ -1109,14 +1109,28 @@ def updates_an_input(program):
 
 
 class TunedPlan(Plan):
-    """Several fitting plans; each bound call picks the fastest with ``AutoTuner``."""
+    """Several fitting plans; each bound call picks the fastest with ``AutoTuner``.
+
+    Before the forced configurations of a family comes the library's own choice (configuration
+    0), which may be a kernel that none of them forces: 16-bit products through a workspace, the
+    im2col path, the key-streaming attention, the held softmax."""
 
     family = "tuned"
 
     def __init__(self, plans, namespace):
+        forced = next((i for i, p in enumerate(plans) if getattr(p, "config", 0)), None)
+        if forced is not None:
+            plans = [*plans[:forced], plans[forced].with_config(0), *plans[forced:]]
         self.plans = plans
         self.namespace = namespace
         self.chosen = {}
+
+    @staticmethod
+    def _described(plan):
+        described = plan.describe()
+        if getattr(plan, "config", None) == 0:
+            described["config"] = 0
+        return described
 
     def bind(self, values, index):
         import json
@@ -1130,7 +1144,7 @@ class TunedPlan(Plan):
             except (LoweringError, TypeError, ValueError):
                 continue
             bound.append(launch)
-            keys.append(json.dumps(plan.describe(), sort_keys=True, default=str))
+            keys.append(json.dumps(self._described(plan), sort_keys=True, default=str))
         if not bound:
             raise LoweringError("no candidate kernel accepts these arguments")
         if len(bound) == 1:
@@ -1144,7 +1158,7 @@ class TunedPlan(Plan):
         return bound[best]
 
     def describe(self):
-        return {"family": "tuned", "candidates": [p.describe() for p in self.plans],
+        return {"family": "tuned", "candidates": [self._described(p) for p in self.plans],
                 "chosen": sorted(set(self.chosen.values()))}
 
 

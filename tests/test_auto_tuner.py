@@ -356,3 +356,39 @@ def test_tuned_softmax_and_pool_pick_a_kernel():
     assert torch.equal(yo, F.max_pool2d(xi, (2, 2)))
     (plan,) = pool.plans()
     assert plan["family"] == "tuned" and len(plan["chosen"]) == 1
+
+
+def test_tuned_calls_time_the_library_choice():
+    import functools
+
+    f16 = functools.partial(torch.empty, dtype=torch.float16)
+    pool = functools.partial(pg.max_pool2d_arrangement, ceil_mode=False)
+    cases = (
+        (ninetoothed.make(pg.matmul_arrangement, pg.matmul_application, pg.matmul_tensors()),
+         (f16(100, 99), f16(99, 70), f16(100, 70)), {}),
+        (pg.make_conv2d(), (f16(2, 64, 7, 7), f16(96, 64, 3, 3), f16(2, 96, 7, 7)), {"padding_h": 1, "padding_w": 1}),
+        (ninetoothed.make(pg.attention_arrangement, pg.attention_application_scaled, pg.attention_tensors()),
+         (f16(1, 2, 1, 128), f16(1, 2, 512, 128), f16(1, 2, 512, 128), False, f16(1, 2, 1, 128)), {}),
+        (pg.make_softmax(), (f16(8, 30000), f16(8, 30000)), {"BLOCK_SIZE": 30000}),
+        (ninetoothed.make(pool, pg.max_pool2d_application, pg.max_pool2d_tensors()),
+         (f16(2, 3, 16, 16), f16(2, 3, 8, 8)), {"WINDOW_HEIGHT": 2, "WINDOW_WIDTH": 2}),
+    )
+    for handle, args, meta in cases:
+        public = dict(zip(handle._kernel.params, args))
+        tuned = handle._kernel.specialize(public, meta, tune=True).describe()
+        configs = [c.get("config") for c in tuned["candidates"] if c["family"] != "generic"]
+        assert tuned["family"] == "tuned" and configs[0] == 0 and configs[1:] == sorted(configs[1:]) and 0 not in configs[1:]
+
+
+@pytest.mark.gpu
+def test_tuned_products_of_unaligned_operands():
+    # Of the forced configurations only the element-wise loader takes these; the library's own
+    # choice, copies in aligned rows, is tens of times faster and so the one that is kept.
+    h = ninetoothed.make(pg.matmul_arrangement, pg.matmul_application, pg.matmul_tensors(), max_num_configs=4)
+    g = torch.Generator().manual_seed(9)
+    a, b = (torch.randn(*s, generator=g).half().cuda() for s in ((644, 3803), (3803, 3434)))
+    out = torch.empty(644, 3434, dtype=torch.float16, device="cuda")
+    h(a, b, out)
+    assert torch.allclose(out.double(), a.double() @ b.double(), atol=0.25, rtol=2e-3)  # rounding at up to 256
+    (plan,) = h.plans()
+    assert '"config": 0' in plan["chosen"][0]
