@@ -948,13 +948,20 @@ class _TileEmitter(_Emitter):
 
     def vector_context(self, root, coords, tag, var, width):
         """``context`` for a loop over vectors of ``width``: (lines ahead of the elements, lines
-        per element ``u``, (tensor, head) of each load that reads vectors)."""
-        self.vec, self.var, self.pre, self.vectors = width, var, [], []
+        per element ``u``, (tensor, head) of each load that reads vectors); None where an element
+        is looked up in a table, whose lanes then read ``width`` entries apart (bf16 norm of [4096,
+        1000] cut from wider rows, two rows a tile: 49.4 us so, 26.8 element by element)."""
+        self.vec, self.var, self.pre, self.vectors, self.tabled = width, var, [], [], False
         try:
             lines = self.context(root, coords, tag)
-            return self.pre, lines, self.vectors
+            return None if self.tabled else (self.pre, lines, self.vectors)
         finally:
             self.vec = 0
+
+    def look_up(self, lin):
+        """Note that element ``lin`` of a table is read."""
+        if self.vec and re.search(rf"\b{self.var}\b", lin):
+            self.tabled = True
 
     def _canon(self, v, coords):
         return tuple("0" if size == 1 else c for size, c in zip(self.shapes[id(v)], coords))
@@ -1020,6 +1027,8 @@ class _TileEmitter(_Emitter):
                 self.define(v, t, f"(({w}){ld.format(f'{vec}.e[u]')})", exact=True)
                 self.masks[id(v)] = frozenset()
                 return
+            if name not in self.plan.forms:
+                self.look_up(lin)
             entry = self.plan.level_index(name, ks, lin, self)
             ix = f"{self.tag}x{len(self.names)}"
             self.lines.append(f"      const int {ix} = {entry};")
@@ -1037,6 +1046,7 @@ class _TileEmitter(_Emitter):
         if op == "offsets":
             name, d = args[0].args[0], int(args[1])
             lin = _ravel(self.coords[id(v)], self.shapes[id(v)])
+            self.look_up(lin)
             self.names[id(v)] = f"(long long)f_{name}_{d}[pbo_{name}_{d} + {lin}]"
             self.types[id(v)] = "int32"
             self.masks[id(v)] = frozenset()
@@ -1617,7 +1627,8 @@ class TilePlan(GenericPlan):
         first, loops = "0", []
         width = self._vector_width(em)
         if width and extent >= width:
-            pre, each, vectors = em.vector_context(operand, coords, f"w{k}_", "l", width)
+            found = em.vector_context(operand, coords, f"w{k}_", "l", width)
+            pre, each, vectors = found or ([], [], [])
             if vectors:
                 bound, first = self._vector_bound(vectors, extent, width, f"n{k}")
                 loops += [
@@ -1800,8 +1811,11 @@ class TilePlan(GenericPlan):
 
         lines, first = [], "0"
         width = self._vector_width(em) if vectors and self.forms.get(out, (0, None))[0] == 1 else 0
-        if width and n_tile >= width:
-            pre, each, read = em.vector_context(v, coords, f"z{out}_", "j", width)
+        found = em.vector_context(v, coords, f"z{out}_", "j", width) if width and n_tile >= width else None
+        if found is not None and not found[2] and n_tile < 256 * width:
+            found = None  # results of reductions alone, which fewer lanes would write (0.2 us more at 33 columns)
+        if found is not None:
+            pre, each, read = found
             bound, first = self._vector_bound(read + [(out, "")], n_tile, width, f"n_{out}")
             lines += [
                 f"    {{  // `{out}`, {width} elements per lane",
@@ -1829,7 +1843,7 @@ class TilePlan(GenericPlan):
                 f"      p_{out}[oi] = {stored()};",
                 "    }",
             ]
-        if width and n_tile >= width:
+        if found is not None:
             lines.append("    }")
         return "\n".join(lines)
 

@@ -215,3 +215,15 @@ def test_lds_of_a_whole_workgroup_reduction_is_counted(width, whole_workgroup):
     declared = sum(4 * int(n) for n in re.findall(r"__shared__ float \w+\[(\d+)\]", "\n".join(plan.decls)))
     assert declared == plan.lds_bytes <= 64 * 1024
     assert ("red0_w" in "\n".join(plan.decls)) == whole_workgroup
+
+
+@pytest.mark.parametrize("x, vectors", ((torch.empty(6, 64), True), (torch.empty(6, 70)[:, 3:67], False),
+                                        (torch.empty(64, 6).t(), False)))
+def test_vectors_only_without_tables(x, vectors):
+    # Tiles of several rows of a wider or transposed tensor keep their tables, and with them one
+    # lane an element: lanes that took vectors would read a table's entries apart from each other.
+    handle = _handle("centred")
+    values = dict(zip(handle._abi["public_args"], (x, torch.empty(6, 64))))
+    plan = handle._kernel.specialize(values, {"ROWS": 4, "WIDTH": 64})
+    body = plan.sources_for(values)[0].split("nt_generic_tile(")[1]
+    assert ("nt_ldv" in body) == ("nt_stv" in body) == vectors
