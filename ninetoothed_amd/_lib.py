@@ -103,7 +103,7 @@ _SIGNATURES = {
     "nt_rtc_launch": (_P, ctypes.c_uint32, ctypes.c_uint32, ctypes.POINTER(_P), _P),
 }
 _RESTYPES = {"nt_conv2d_workspace_size": ctypes.c_int64, "nt_attention_workspace_size": ctypes.c_int64,
-             "nt_gemm_workspace_size": ctypes.c_int64,              "nt_rtc_free": None}
+             "nt_gemm_workspace_size": ctypes.c_int64, "nt_rtc_free": None}
 
 _lock = threading.Lock()
 _library = None

@@ -1652,7 +1652,11 @@ static bool b_tail_zero(int64_t K, int64_t sb_k, int64_t N) { return (K % 32 == 
 //   - an out that the 128-wide kernel's epilogue cannot store, through the fp32 partials.
 // bf16 us with weights rotated past the caches, split / before / torch: 200 x 4096 x 4096 22.8 /
 // 51.3 / 22.2, 128 x 4096 x 4096 19.2 / 52.9 / 24.0, 200 x 4096 x 11008 45.2 / 130 / 48.9,
-// 512 x 4096 x 4096 36.5 / 52.5 / 29.7, 1000 x 1024 x 4096 20.8 / 36.1 / 18.7.
+// 512 x 4096 x 4096 36.5 / 52.5 / 29.7, 1000 x 1024 x 4096 20.8 / 36.1 / 18.7.  K below 96 costs a
+// copy and up to twelve times the products, and is still the faster (us, copied / before): whole
+// tiles of K = 64, which the register-staged kernel takes, 4096 x 4096 13.0 / 17.2, 1024 x 1024
+// 7.3 / 14.0, 262144 x 256 57.0 / 60.6; on the element-wise loader 4096 x 4096 x 8 13.0 / 65.8,
+// 262144 x 64 x 8 61.8 / 303, 100 x 4096 x 88 7.1 / 90.7.
 struct Gemm16Route {
   bool bt, pad_a, pad_b, big, part;
   int64_t Kp, Nbp, splits, per;          // K as multiplied; a padded b's row length

@@ -310,7 +310,7 @@ __global__ __launch_bounds__(NT) void softmax_long_kernel(const typename elem<T>
 // in place of the elements; 16-bit elements stay raw, their exponentials computed twice.
 // HBM-bound where there are segments enough; with few, one CU's fetch rate and the latency of
 // the three phases.  Measured against the two-sweep kernel, which fetches the segment twice:
-// fp32 [32, 50257] 13.2 -> 9.3 us, [2048, 50257] 229 -> 161 (5.1 TB/s), fp16 [2048, 50257]
+// fp32 [32, 50257] 12.9 -> 8.8 us, [2048, 50257] 229 -> 161 (5.1 TB/s), fp16 [2048, 50257]
 // 103 -> 77; against the register path's element loads: bf16 [4096, 5001] 59.5 -> 19.8, fp16
 // [4096, 16001] 179 -> 42, fp32 [32, 12345] 7.9 -> 4.7.
 template <typename T, int NT, int R>
@@ -321,7 +321,8 @@ __global__ __launch_bounds__(NT) void softmax_hold_kernel(const typename elem<T>
   constexpr int V = 16 / sizeof(S);
   constexpr uint32_t NEG = elem<T>::code == NT_DTYPE_F32 ? 0xff800000u : elem<T>::code == NT_DTYPE_F16 ? 0xfc00fc00u : 0xff80ff80u;
   // Widened 16-bit elements are kept from one phase to the next where they fit (bf16
-  // [4096, 5001]: 19.8 us, widened anew 22.8); at 1024 lanes and R = 16 they would spill.
+  // [4096, 5001]: 19.8 us, widened anew 22.8); at 1024 lanes and R = 16 they would spill (55
+  // registers of the 128 a lane has; widened anew it takes 98).
   constexpr bool ANEW = NT == 1024 && R == 16;
   __shared__ float red[NT / 64];
   const int64_t seg = blockIdx.x;

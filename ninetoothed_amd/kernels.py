@@ -145,8 +145,8 @@ def add(lhs, rhs, out):
 # workgroups of four, eight or one wave (the reference's num_warps candidates 4, 8, 1), the
 # two-sweep kernel, the lane-group kernel, the element-wise kernel.
 SOFTMAX_CONFIGS = (1, 2, 3, 4, 5, 6)
-# SOFTMAX_FORCED adds the held kernel of 256 and of 1024 lanes, which config 0 takes and
-# the tuner does not time.
+# SOFTMAX_FORCED adds the held kernel of 256 and of 1024 lanes, which the tuner times as
+# config 0.
 SOFTMAX_FORCED = SOFTMAX_CONFIGS + (7, 8)
 SOFTMAX_ANY = 6  # the configuration that takes any strides and any output dtype
 
@@ -415,7 +415,7 @@ def conv2d_workspace_bytes(x, w, padding=(0, 0)):
 # tiles, the input read in place by the 224-position strip kernel (only the filter re-laid),
 # 1 x 1 filters as a batch of products on the 128 x 128-tile GEMM kernel, re-laid input
 # through the DMA kernel of 128 x 128 tiles.  CONV_FORCED adds the im2col matrix written out
-# with the filter in place, which config 0 takes for small planes and the tuner does not time.
+# with the filter in place, which config 0 takes for small planes (and the tuner times as such).
 CONV_CONFIGS = (1, 2, 3, 4, 5, 6, 7)
 CONV_FORCED = CONV_CONFIGS + (8,)
 
@@ -482,10 +482,10 @@ def conv2d(x, w, y, padding=(0, 0), stride=(1, 1), dilation=(1, 1), round_dtype=
 
 # ------------------------------------------------------------------- attention
 # Kernel configurations of the 16-bit attention that ``config`` can force (0: the key-streaming
-# kernel for few queries or few heads, else the eight-wave kernel where its conditions hold):
+# kernel for few queries or few heads over enough keys, else the eight-wave kernel where its conditions hold):
 # the one-wave-per-SIMD pipelined kernel (head dim 128), the eight-wave kernel, the four-wave
-# kernels (any strides).  ATTENTION_FORCED adds the key-streaming kernel (whose keys config 0
-# may also split over workgroups, through a workspace), which the tuner does not time.
+# kernels (any strides).  ATTENTION_FORCED adds the key-streaming kernel, which the tuner times
+# as config 0 (where its keys may also be split over workgroups, through a workspace).
 ATTENTION_CONFIGS = (1, 2, 3)
 ATTENTION_FORCED = ATTENTION_CONFIGS + (4,)
 

@@ -7,7 +7,9 @@ fp32, as the north-star contract states; attention in fp32 keeps the reference
 test's 0.025 (tests/test_attention.py:99-117 of the reference).
 """
 
+import ctypes
 import math
+import struct
 
 import pytest
 import torch
@@ -569,9 +571,21 @@ def test_gemm_few_rows_walking_columns(mnk, dtype):
     (3001, 4099, 131), (4096, 2816, 97)))  # ... on 256 x 256 tiles
 def test_gemm_through_a_workspace(mnk, bt, dtype):
     # The workspace route (split reduction, padded copies of unaligned operands, an out the
-    # 128-wide epilogue cannot store) against fp64 and against the same call with none.  Rows
-    # start off 16-byte boundaries and are followed by infinities, which no product may see.
+    # 128-wide epilogue cannot store) against fp64 and against the same call with none (the C
+    # entry that takes none).  Rows start off 16-byte boundaries and are followed by infinities,
+    # which no product may see.  Few rows against b^T take a kernel that needs no workspace.
     m, n, k = mnk
+    lib = _lib.load()
+
+    def packed(a, b, out, nbytes=0):
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+        v = (ctypes.c_int64 * 24)(0 if dtype == torch.float16 else 1, a.data_ptr(), *a.stride(), b.data_ptr(), *b.stride(),
+                                  0, 0, 0, out.data_ptr(), *out.stride(), _lib.dtype_code(out.dtype), m, n, k, one, 0,
+                                  _lib.DTYPE_NONE, 0, torch.cuda.current_stream().cuda_stream,
+                                  ws.data_ptr() if nbytes else 0, nbytes)
+        return v, ws
+
+    one = struct.unpack("<I", struct.pack("<f", 1.0))[0]
     inf = float("inf")
     abuf = torch.full((m, k + 3), inf, dtype=dtype, device=DEV)
     a = abuf[:, 1:k + 1] if k % 8 else abuf[:, :k].contiguous()
@@ -595,6 +609,16 @@ def test_gemm_through_a_workspace(mnk, bt, dtype):
     out = torch.empty((m, n), dtype=dtype, device=DEV)
     kernels.gemm(a, b, out)
     assert torch.allclose(out.double(), ref, atol=tol, rtol=tol)
+    nbytes = lib.nt_gemm_workspace_size(packed(a, b, out)[0])
+    assert (nbytes > 0) == (not (bt and m <= 64))
+    with_ws, without, short = (torch.full_like(out, 7.0) for _ in range(3))
+    v, ws = packed(a, b, with_ws, nbytes)
+    assert lib.nt_gemm_packed_ws(v) == 0
+    assert lib.nt_gemm_packed(packed(a, b, without)[0]) == 0
+    u, ws2 = packed(a, b, short, max(nbytes - 256, 0))  # too little: as without
+    assert lib.nt_gemm_packed_ws(u) == 0
+    assert torch.equal(with_ws, out) and torch.equal(short, without)
+    assert torch.allclose(without.double(), ref, atol=tol, rtol=tol)
 
 
 def test_gemm_few_rows_rejects_unfit_calls():
@@ -1405,7 +1429,7 @@ def test_attention_pipe_bf16_against_eight_wave(causal):
     (1, 3, 5, 4097, 64), (1, 8, 2, 9000, 128), (3, 16, 32, 1056, 40)))
 def test_attention_few_queries(b, h, sq, sk, d, dtype):
     # The key-streaming kernel: forced, by default without a workspace (C ABI) and by default
-    # with one (its keys split over workgroups from 2,048 keys on), strided K and V, ragged
+    # with one (its keys split over workgroups from 64 tiles of 32 on), strided K and V, ragged
     # key tiles, waves without a tile; scores that rise along the keys, so that every wave
     # and split ends with a max of its own.
     u = _randn((d,), torch.float32, 120) / math.sqrt(d)
@@ -1417,6 +1441,8 @@ def test_attention_few_queries(b, h, sq, sk, d, dtype):
     v.copy_(_randn((b, h, sk, d), dtype, 123))
     qs = kernels.LOG2E / math.sqrt(d)
     tol = 1e-2 if dtype == torch.float16 else 2e-2
+    wanted = _lib.load().nt_attention_workspace_size(b, h, sq, sk, d, 0, _lib.dtype_code(dtype))
+    assert (wanted > 0) == (sk > 63 * 32)  # two splits of 32 tiles or more
     for causal in (False, True):
         ref = _attention_ref64(q, k, v, causal, qs)
         for config in (0, 4):
