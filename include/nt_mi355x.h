@@ -251,7 +251,8 @@ int nt_gemm_packed(const int64_t* v);
  * nt_gemm_packed): v[22] the workspace (256-byte aligned), v[23] its bytes.  It holds fp32
  * partials where few output tiles make the reduction worth splitting, and aligned copies of
  * operands whose rows are not 16-byte aligned or whose K (or a row-major b's N) is no multiple
- * of 8; nothing between calls.  nt_gemm_workspace_size gives the bytes the packed call v[0..21]
+ * of 8, K is below 96, or a row-major b's rows overlap; nothing between calls.
+ * nt_gemm_workspace_size gives the bytes the packed call v[0..21]
  * wants (0: none; the data pointers count, for their alignment); with fewer the call runs as
  * nt_gemm_packed. */
 int64_t nt_gemm_workspace_size(const int64_t* v);
